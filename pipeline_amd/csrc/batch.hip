@@ -6,16 +6,24 @@
 //
 // Work decomposition: a group is split into tiles of 64*K objects.  A work item
 // is (tile, slice of the frusta paired with the tile's group).  A wave owns one
-// item at a time: every lane builds the OBBs of its K objects once (one read of
-// each object's matrix and box), then loops over the item's frusta.  Each
-// frustum's matrix is wave-uniform, so it is read through the scalar cache into
-// SGPRs and feeds the VALU multiplies directly; each (frustum, 64 objects)
-// result is one ballot, stored as one 64-bit mask word by lane 0.  No two items
+// item at a time: every lane builds what the quick test needs of its K objects
+// once (one read of each object's matrix and box), then the wave loops over the
+// item's frusta.  Each frustum's matrix is wave-uniform, so it is read through
+// the scalar cache into SGPRs and feeds the VALU directly; each (frustum, 64
+// objects) result is one lane mask, stored as one 64-bit mask word.  No two items
 // write the same mask word, so no atomics touch the output.
+//
+// What bounds it: with many frusta per object, vector instructions: 60 per
+// frustum and 64 objects with the quick test (55 with two objects per lane), 190
+// when each pair took the exact test.  500,003 objects x 32 frusta, two objects per lane: 109 -> 47 us;
+// 64 frusta over 64 groups of 2,097,152 objects: 40 -> 36 us, 4.5 TB/s, now bound
+// by reading the objects.
 //
 // Schedule: items are sorted by cost (frusta x objects) on the host, and the
 // persistent grid walks them round-robin (wave w takes w, w+W, ...), which
-// bounds the load imbalance by the cost of one item.
+// bounds the load imbalance by the cost of one item.  Objects are not loaded
+// ahead of the item that is tested: without the 22 registers that takes, seven
+// waves run per SIMD instead of five, and hide the loads themselves.
 #include <algorithm>
 #include <cstring>
 #include <numeric>
@@ -68,9 +76,74 @@ __device__ __forceinline__ void load_vp(const float* __restrict__ vps, uint32_t 
   for (int c = 0; c < 16; ++c) vp.m[c] = vps[16 * static_cast<size_t>(frustum) + c];
 }
 
+// Pairs (object, frustum) that the quick test left undecided wait in LDS, one
+// queue per wave, until its entries nearly fill the wave: then each lane takes
+// one of them through the exact test.  A few lanes in a thousand are undecided,
+// which would otherwise send every third wave through the exact test for the
+// sake of one lane.  The mask words they belong to wait with them and are stored
+// once, complete.
+struct QueueEntry {
+  uint32_t object_lo;
+  uint32_t object_hi;  // bits 0-15; bits 16-23: which of the waiting words; bits 24-29: the object's bit in it
+  uint32_t frustum;
+  uint32_t scene;
+};
+struct QueueWord {
+  unsigned long long bits;
+  uint64_t index;  // word of the mask buffer
+};
 template <int K>
-__device__ __forceinline__ void load_item(const SceneDev* __restrict__ scenes, const WorkItem& item, uint32_t lane,
-                                          Slot (&slot)[K], RawObj (&raw)[K])
+struct Queue {
+  static constexpr uint32_t kCapacity = kWave * K;  // any one (frustum, work item) fits when it is empty
+  QueueEntry entry[kCapacity];
+  QueueWord word[kCapacity];
+};
+
+// Orders a wave's LDS accesses across its lanes (they execute in order; the
+// compiler must not move them).
+__device__ __forceinline__ void wave_lds_order()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The exact test of the queue's n entries, then the stores of its n_words words.
+template <int K>
+__device__ __forceinline__ void drain(Queue<K>& queue, uint32_t n, uint32_t n_words, uint32_t lane,
+                                      const SceneDev* __restrict__ scenes, const float* __restrict__ vps,
+                                      unsigned long long* __restrict__ masks)
+{
+  wave_lds_order();
+  for (uint32_t q0 = 0; q0 < n; q0 += kWave) {
+    const bool on = q0 + lane < n;
+    const QueueEntry e = queue.entry[on ? q0 + lane : q0];
+    const SceneDev sc = scenes[e.scene];
+    const size_t object = (static_cast<size_t>(e.object_hi & 0xFFFFu) << 32) | e.object_lo;
+    const Slot slot = make_slot(object, object + 1, sc.xform, sc.ld);
+    const RawObj raw = load_raw(sc.box_a, sc.box_b, sc.planes, sc.ld, slot.i, slot.m);
+    Mat16 m;
+    load_vp(vps, e.frustum, m);
+    if (on & obb_visible(obb_of(raw), m.m))
+      __hip_atomic_fetch_or(&queue.word[(e.object_hi >> 16) & 0xFFu].bits, 1ull << (e.object_hi >> 24),
+                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  }
+  wave_lds_order();
+  for (uint32_t w = lane; w < n_words; w += kWave) masks[queue.word[w].index] = queue.word[w].bits;
+  wave_lds_order();
+}
+
+// What a wave keeps of the work item it tests.
+template <int K>
+struct TileObjects {
+  QuickObj quick[K];
+  unsigned long long tested[K];  // lanes that hold an object with a matrix
+  unsigned long long always[K];  // lanes whose object is visible whatever the frustum (matrix index outside the array)
+};
+
+// The loads of a work item's objects, and what the wave keeps of them.
+template <int K>
+__device__ __forceinline__ void load_objects(const SceneDev* __restrict__ scenes, const WorkItem& item, uint32_t lane,
+                                             Slot (&slot)[K], RawObj (&raw)[K])
 {
   const SceneDev sc = scenes[item.scene];
   const size_t end = item.first_object + item.count;
@@ -81,82 +154,137 @@ __device__ __forceinline__ void load_item(const SceneDev* __restrict__ scenes, c
   }
 }
 
-// The wave-uniform loop state is software-pipelined twice: the objects of the
-// next work item are loaded (vector memory) while the current item is tested,
-// and the next frustum matrix is loaded (scalar memory) while the current one is
-// in use.  Both prefetches are unconditional (indices clamped to the last item
-// or frustum), so no wait lands in front of the FP32 work.
-// Tests a work item's objects (slot, o) against its frusta and stores one mask
-// word per frustum and 64 objects.  The frusta take turns in two sets of scalar
-// registers: while one frustum is tested, the next one's matrix is loaded into
-// the other set (no register copies between frusta).  Every lane stores the
-// wave's mask word (the same value to the same address): a store from lane 0
-// alone would change the exec mask around it, scalar instructions in a loop
-// whose scalar work is a bound.
 template <int K>
-__device__ __forceinline__ void test_frusta(const WorkItem& item, const Slot (&slot)[K], const Obb (&o)[K],
-                                            const KPair* __restrict__ pairs, const float* __restrict__ vps,
-                                            unsigned long long* __restrict__ masks)
+__device__ __forceinline__ void quick_objects(const Slot (&slot)[K], const RawObj (&raw)[K], TileObjects<K>& t)
 {
-  auto test = [&](const KPair& q, const Mat16& m) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const bool vis = slot_visible(slot[k], obb_visible(o[k], m.m));
-      const unsigned long long bits = __ballot(vis);
-      // (a work item holds at least one object: the first word is always stored)
-      if (k == 0 || static_cast<uint32_t>(kWave * k) < item.count) masks[q.mask_word + item.tile_word + k] = bits;
-    }
-  };
-  const uint32_t last = item.pair_count ? item.pair_count - 1 : 0;  // (no item is made without pairs)
-  auto pair_at = [&](uint32_t p) { return pairs[item.pair_begin + (p < last ? p : last)]; };
-  KPair pa = pair_at(0), pb;
-  Mat16 va, vb;
-  load_vp(vps, pa.frustum, va);
-  for (uint32_t p = 0; p < item.pair_count; p += 2) {
-    pb = pair_at(p + 1);
-    load_vp(vps, pb.frustum, vb);
-    test(pa, va);
-    if (p + 1 >= item.pair_count) break;
-    pa = pair_at(p + 2);
-    load_vp(vps, pa.frustum, va);
-    test(pb, vb);
+  for (int k = 0; k < K; ++k) {
+    t.quick[k] = quick_of(obb_of(raw[k]));
+    t.tested[k] = ballot(slot[k].valid & !slot[k].bad_matrix);
+    t.always[k] = ballot(slot[k].valid & slot[k].bad_matrix);
   }
 }
 
-template <int K>
+// Tests a work item against its frusta, one mask word per frustum and 64
+// objects.  Words that the quick test (quick_cull.hpp) decides whole are stored
+// at once, by every lane (the same value to the same address: a store from lane
+// 0 alone would change the exec mask around it); the others wait in the queue.
+// view_of(p, frustum, m) gives the QuickView of the item's p-th frustum; with
+// `last` the queue is drained before the return.
+template <int K, class ViewOf>
+__device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObjects<K>& t, uint32_t lane,
+                                            const KPair* __restrict__ pairs, const SceneDev* __restrict__ scenes,
+                                            const float* __restrict__ vps, unsigned long long* __restrict__ masks,
+                                            Queue<K>& queue, uint32_t& waiting, uint32_t& words, bool last,
+                                            ViewOf&& view_of)
+{
+  const KPair* const list = pairs + item.pair_begin;
+  uint32_t p = 0;
+  KPair next = list[0];  // (no item is made without pairs)
+  for (;;) {
+    bool full = false;
+    while (p < item.pair_count) {
+      const KPair q = next;
+      Mat16 m;
+      load_vp(vps, q.frustum, m);
+      const QuickView view = view_of(p, q.frustum, m);
+      next = list[p + 1 < item.pair_count ? p + 1 : p];
+      unsigned long long bits[K], open[K];
+      uint32_t n_open = 0;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const QuickResult<unsigned long long> r = quick_wave(t.quick[k], m.m, view);
+        bits[k] = (r.visible & t.tested[k]) | t.always[k];
+        open[k] = t.tested[k] & ~(r.visible | r.culled);
+        n_open += static_cast<uint32_t>(__builtin_popcountll(open[k]));
+      }
+      const uint64_t word = q.mask_word + item.tile_word;
+      if (n_open == 0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+          // (a work item holds at least one object: the first word is always stored)
+          if (k == 0 || static_cast<uint32_t>(kWave * k) < item.count) masks[word + k] = bits[k];
+      } else {
+        full = waiting + n_open > Queue<K>::kCapacity;
+        if (full) {  // this frustum again, once the queue is empty
+          next = q;
+          break;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (k != 0 && static_cast<uint32_t>(kWave * k) >= item.count) continue;
+          if (open[k] == 0) {
+            masks[word + k] = bits[k];
+            continue;
+          }
+          if ((open[k] >> lane) & 1) {
+            const uint64_t object = item.first_object + lane + kWave * k;
+            const uint32_t at = waiting + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(open[k] >> 32),
+                                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(open[k]), 0u));
+            queue.entry[at] = QueueEntry{static_cast<uint32_t>(object),
+                                         static_cast<uint32_t>(object >> 32) | (words << 16) | (lane << 24), q.frustum,
+                                         item.scene};
+          }
+          if (lane == 0) queue.word[words] = QueueWord{bits[k], word + k};
+          waiting += static_cast<uint32_t>(__builtin_popcountll(open[k]));
+          ++words;
+        }
+      }
+      ++p;
+    }
+    if (full | last) {
+      drain<K>(queue, waiting, words, lane, scenes, vps, masks);
+      waiting = words = 0;
+    }
+    if (!full) break;
+  }
+}
+
+// The QuickViews of a launch's frusta, computed once per workgroup into LDS
+// (Table: at most kTableViews frusta, 6 KB; else each use computes its own).
+// From the matrix in scalar registers a QuickView takes 34 vector and 18 scalar
+// instructions per use, from LDS three broadcast reads.
+constexpr uint32_t kTableViews = 128;
+constexpr uint32_t kBatchWaves = 4;  // waves of a workgroup, at most
+
+template <int K, bool Table>
 __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restrict__ items, uint32_t n_items,
                                                          const KPair* __restrict__ pairs,
                                                          const SceneDev* __restrict__ scenes,
-                                                         const float* __restrict__ vps,
+                                                         const float* __restrict__ vps, uint32_t n_frusta,
                                                          unsigned long long* __restrict__ masks)
 {
+  __shared__ QuickView table[Table ? kTableViews : 1];
+  __shared__ Queue<K> queues[kBatchWaves];
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t waves_per_block = blockDim.x / kWave;
   const uint32_t n_waves = gridDim.x * waves_per_block;
-  uint32_t it = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_block + threadIdx.x / kWave);
-  if (it >= n_items) return;
-  WorkItem item = items[it];
-  Slot slot[K];
-  RawObj raw[K];
-  load_item<K>(scenes, item, lane, slot, raw);
-  for (;;) {
-    const uint32_t nit = it + n_waves;
-    const WorkItem next_item = items[nit < n_items ? nit : it];
-    Slot next_slot[K];
-    RawObj next_raw[K];
-    load_item<K>(scenes, next_item, lane, next_slot, next_raw);
-    Obb o[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) o[k] = obb_of(raw[k]);
-    test_frusta<K>(item, slot, o, pairs, vps, masks);
-    if (nit >= n_items) break;
-    it = nit;
-    item = next_item;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      slot[k] = next_slot[k];
-      raw[k] = next_raw[k];
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  uint32_t it = blockIdx.x * waves_per_block + wave;
+  uint32_t waiting = 0, words = 0;
+  auto view_of = [&](uint32_t, uint32_t f, const Mat16& m) { return Table ? table[f] : quick_view(m.m); };
+  for (bool first = true;; first = false) {
+    const WorkItem item = items[it < n_items ? it : 0];  // (n_items >= 1)
+    Slot slot[K];
+    RawObj raw[K];
+    load_objects<K>(scenes, item, lane, slot, raw);
+    if (first) {  // the table is built while the first objects are in flight
+      if (Table) {
+        for (uint32_t f = threadIdx.x; f < n_frusta; f += blockDim.x) {
+          Mat16 m;
+          load_vp(vps, f, m);
+          table[f] = quick_view(m.m);
+        }
+        lds_barrier();
+      }
+      if (it >= n_items) return;  // (a wave without an item helped with the table)
     }
+    TileObjects<K> objects;
+    quick_objects<K>(slot, raw, objects);
+    const bool last = it + n_waves >= n_items;
+    test_frusta<K>(item, objects, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, last, view_of);
+    if (last) break;
+    it += n_waves;
   }
 }
 
@@ -166,6 +294,9 @@ __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restr
 // without a per-batch item list: a tile of entry a costs pair_count(a), every
 // wave takes the tiles whose cost prefix falls in its equal share of the total
 // cost, and walks them in order (the entry changes at most n_entries times).
+
+constexpr uint32_t kServeViews = 64;  // frusta of a request, at most (dpc_server_submit)
+static_assert(kServeViews <= kWave, "one lane per frustum");
 
 template <int K>
 __device__ __forceinline__ WorkItem serve_item(const ServeEntry& e, uint32_t tile)
@@ -189,10 +320,13 @@ __global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __res
                                                          const float* __restrict__ vps,
                                                          unsigned long long* __restrict__ masks)
 {
+  __shared__ Queue<K> queues[kBatchWaves];
+  __shared__ QuickView views[kBatchWaves][kServeViews];  // of the wave's current entry
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t waves_per_block = blockDim.x / kWave;
   const uint64_t W = static_cast<uint64_t>(gridDim.x) * waves_per_block;
-  const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_block + threadIdx.x / kWave);
+  const uint32_t block_wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t wave = static_cast<uint64_t>(blockIdx.x) * waves_per_block + block_wave;
   const uint64_t c0 = total_cost * wave / W, c1 = total_cost * (wave + 1) / W;
   if (c0 >= c1) return;
   // first tile whose cost start is >= c0
@@ -211,9 +345,7 @@ __global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __res
   auto cost_start = [](const ServeEntry& ent, uint64_t tile) { return ent.cost_begin + tile * ent.pair_count; };
   if (t >= e.tiles || cost_start(e, t) >= c1) return;
   WorkItem item = serve_item<K>(e, static_cast<uint32_t>(t));
-  Slot slot[K];
-  RawObj raw[K];
-  load_item<K>(scenes, item, lane, slot, raw);
+  uint32_t waiting = 0, words = 0, viewed = ~0u;
   for (;;) {
     // the next tile of this wave (or the current one again, as a harmless prefetch target)
     ServeEntry ne = e;
@@ -222,23 +354,28 @@ __global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __res
     advance(ne, na, nt);
     const bool more = nt < ne.tiles && cost_start(ne, nt) < c1;
     const WorkItem next_item = more ? serve_item<K>(ne, static_cast<uint32_t>(nt)) : item;
-    Slot next_slot[K];
-    RawObj next_raw[K];
-    load_item<K>(scenes, next_item, lane, next_slot, next_raw);
-    Obb o[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) o[k] = obb_of(raw[k]);
-    test_frusta<K>(item, slot, o, pairs, vps, masks);
+    Slot slot[K];
+    RawObj raw[K];
+    load_objects<K>(scenes, item, lane, slot, raw);
+    if (viewed != a) {  // the entry's QuickViews, one per lane, while its first objects are in flight
+      wave_lds_order();
+      if (lane < e.pair_count) {
+        Mat16 m;
+        load_vp(vps, pairs[e.pair_begin + lane].frustum, m);
+        views[block_wave][lane] = quick_view(m.m);
+      }
+      wave_lds_order();
+      viewed = a;
+    }
+    TileObjects<K> objects;
+    quick_objects<K>(slot, raw, objects);
+    test_frusta<K>(item, objects, lane, pairs, scenes, vps, masks, queues[block_wave], waiting, words, !more,
+                   [&](uint32_t p, uint32_t, const Mat16&) { return views[block_wave][p]; });
     if (!more) break;
     e = ne;
     a = na;
     t = nt;
     item = next_item;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      slot[k] = next_slot[k];
-      raw[k] = next_raw[k];
-    }
   }
 }
 
@@ -534,18 +671,20 @@ int dpc_cull_batch(const dpc_batch_plan* plan, const float* d_vps, uint64_t* d_m
   const dim3 grid(static_cast<unsigned>(blocks)), block(c.block_threads);
   auto* m = reinterpret_cast<unsigned long long*>(d_masks);
   hipStream_t s = as_stream(stream);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, plan->d_items, plan->n_items, plan->d_pairs, plan->d_scenes, d_vps,
+                       plan->n_frusta, m);
+  };
+  const bool table = plan->n_frusta <= kTableViews;
   switch (c.objects_per_lane) {
     case 1:
-      hipLaunchKernelGGL(cull_batch_kernel<1>, grid, block, 0, s, plan->d_items, plan->n_items, plan->d_pairs,
-                         plan->d_scenes, d_vps, m);
+      table ? launch(cull_batch_kernel<1, true>) : launch(cull_batch_kernel<1, false>);
       break;
     case 2:
-      hipLaunchKernelGGL(cull_batch_kernel<2>, grid, block, 0, s, plan->d_items, plan->n_items, plan->d_pairs,
-                         plan->d_scenes, d_vps, m);
+      table ? launch(cull_batch_kernel<2, true>) : launch(cull_batch_kernel<2, false>);
       break;
     default:
-      hipLaunchKernelGGL(cull_batch_kernel<4>, grid, block, 0, s, plan->d_items, plan->n_items, plan->d_pairs,
-                         plan->d_scenes, d_vps, m);
+      table ? launch(cull_batch_kernel<4, true>) : launch(cull_batch_kernel<4, false>);
       break;
   }
   return check_launch("cull_batch_kernel");

@@ -10,9 +10,25 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "quick_cull.hpp"
+
 #pragma clang fp contract(off)
 
 namespace dpc {
+
+// The wave's lanes whose condition holds.  (__ballot takes an integer: a
+// condition formed from lane masks is then first spread to a register and
+// compared again.)
+__device__ __forceinline__ unsigned long long ballot(bool v) { return __builtin_amdgcn_ballot_w64(v); }
+
+// Orders LDS stores before the LDS loads that follow it in the workgroup, and
+// nothing else: loads from global memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 // A 4x4 row-major matrix passed by value in kernel arguments: the compiler
 // loads it into scalar registers once per wave, and the VALU multiplies read
@@ -169,6 +185,15 @@ __device__ __forceinline__ bool obb_visible(const Obb& o, const float* vp)
 #pragma unroll
   for (int a = 0; a < 3; ++a) culled = culled | s.lo_all[a] | (s.hi_all[a] & !s.lo_any[a]);
   return !culled;
+}
+
+__device__ __forceinline__ QuickObj quick_of(const Obb& o) { return quick_obj(o.p, o.ex, o.ey, o.ez); }
+
+// The quick test of a wave's objects: lane masks.
+__device__ __forceinline__ QuickResult<unsigned long long> quick_wave(const QuickObj& q, const float* vp,
+                                                                      const QuickView& v)
+{
+  return quick_test<unsigned long long>(q, vp, v, [](float a, float b) { return ballot(a < b); });
 }
 
 // The raw inputs of one object as loaded from the SoA arrays: box (lower.xyz,

@@ -93,18 +93,13 @@ __device__ __forceinline__ void load_level(const float4* __restrict__ L, size_t 
   }
 }
 
-// Orders one level's LDS stores before the next level's LDS loads.  Global
-// memory needs no ordering inside a run: every parent the run reads from memory
-// lies outside the slots the run writes before that read (it was written by an
-// earlier launch, or is an unlisted slot or a slot of a later pass of the same
-// level, whose old value the reference reads too), so the wait covers LDS only
-// and the next level's prefetched loads stay in flight across it.
-__device__ __forceinline__ void lds_barrier()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+// Between levels, lds_barrier orders one level's LDS stores before the next
+// level's LDS loads.  Global memory needs no ordering inside a run: every parent
+// the run reads from memory lies outside the slots the run writes before that
+// read (it was written by an earlier launch, or is an unlisted slot or a slot of
+// a later pass of the same level, whose old value the reference reads too), so
+// the wait covers LDS only and the next level's prefetched loads stay in flight
+// across it.
 
 // A parent that is not staged in LDS, read from memory.  The empty asm takes
 // the loaded values as register operands: it keeps the compiler from folding

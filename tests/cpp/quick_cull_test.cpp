@@ -1,0 +1,199 @@
+// The quick visibility test (pipeline_amd/csrc/quick_cull.hpp) against the
+// oracle's exact test, on the CPU: whatever it decides has to be the oracle's
+// answer, bit for bit.  Objects and matrices of ordinary scenes, boxes that touch
+// planes, magnitudes from denormal to overflow, infinities and NaN, projective
+// object matrices, orthographic, reversed and degenerate view-projections.
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <limits>
+#include <random>
+
+#include "oracle.h"
+#include "quick_cull.hpp"
+
+namespace {
+
+struct V4 {
+  float x, y, z, w;
+};
+
+std::mt19937_64 rng(20260417);
+
+double uniform(double lo, double hi) { return std::uniform_real_distribution<double>(lo, hi)(rng); }
+int pick(int n) { return static_cast<int>(rng() % static_cast<unsigned>(n)); }
+
+const float kOdd[] = {0.0f, -0.0f, 1.0f, -1.0f, 1e-45f, -1e-40f, 0x1p-126f, 0x1p-75f, 0x1p55f, 0x1p56f, -0x1p59f, 0x1p60f,
+                      0x1p63f, 0x1p100f, 3e38f, -3e38f, std::numeric_limits<float>::infinity(),
+                      -std::numeric_limits<float>::infinity(), std::numeric_limits<float>::quiet_NaN()};
+
+// A perspective or orthographic view-projection at a random place.
+void view_projection(float vp[16], bool ortho, bool reversed)
+{
+  double q[4], n = 0;
+  for (double& v : q) {
+    v = uniform(-1, 1);
+    n += v * v;
+  }
+  for (double& v : q) v /= std::sqrt(n);
+  const double x = q[0], y = q[1], z = q[2], w = q[3];
+  const double r[3][3] = {{1 - 2 * (y * y + z * z), 2 * (x * y + z * w), 2 * (x * z - y * w)},
+                          {2 * (x * y - z * w), 1 - 2 * (x * x + z * z), 2 * (y * z + x * w)},
+                          {2 * (x * z + y * w), 2 * (y * z - x * w), 1 - 2 * (x * x + y * y)}};
+  const double eye[3] = {uniform(-50, 50), uniform(-50, 50), uniform(-50, 50)};
+  double view[4][4] = {};
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j) view[i][j] = r[i][j];
+  for (int j = 0; j < 3; ++j) view[3][j] = -(eye[0] * r[0][j] + eye[1] * r[1][j] + eye[2] * r[2][j]);
+  view[3][3] = 1;
+  double p[4][4] = {};
+  const double nr = uniform(0.05, 1), fr = uniform(50, 3000), s = 1 / std::tan(uniform(0.1, 1.2));
+  if (ortho) {
+    p[0][0] = 1 / uniform(10, 500);
+    p[1][1] = 1 / uniform(10, 500);
+    p[2][2] = -2 / (fr - nr);
+    p[3][2] = -(fr + nr) / (fr - nr);
+    p[3][3] = 1;
+  } else {
+    p[0][0] = s / 1.7;
+    p[1][1] = s;
+    p[2][2] = -(fr + nr) / (fr - nr);
+    p[2][3] = -1;
+    p[3][2] = -2 * fr * nr / (fr - nr);
+  }
+  if (reversed)
+    for (int i = 0; i < 4; ++i) p[i][2] = -p[i][2];
+  for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 4; ++j) {
+      double v = 0;
+      for (int k = 0; k < 4; ++k) v += view[i][k] * p[k][j];
+      vp[4 * i + j] = static_cast<float>(v);
+    }
+}
+
+// A world box: point and three edges (xyzw each).
+void object(float obb[16], double extent, double size)
+{
+  for (int c = 0; c < 16; ++c) obb[c] = 0.0f;
+  for (int c = 0; c < 3; ++c) obb[c] = static_cast<float>(uniform(-extent, extent));
+  obb[3] = 1.0f;
+  for (int e = 1; e < 4; ++e)
+    for (int c = 0; c < 3; ++c) obb[4 * e + c] = static_cast<float>(uniform(-size, size));
+}
+
+long failures = 0, decided = 0, pairs = 0;
+
+void check(const float obb[16], const float vp[16], const char* what)
+{
+  V4 v[4];
+  std::memcpy(v, obb, sizeof v);
+  const dpc::QuickObj q = dpc::quick_obj(v[0], v[1], v[2], v[3]);
+  const dpc::QuickView view = dpc::quick_view(vp);
+  const auto r = dpc::quick_test<bool>(q, vp, view, [](float a, float b) { return a < b; });
+  const bool want = orc_is_visible_obb(vp, obb) != 0;
+  ++pairs;
+  if (r.visible || r.culled) ++decided;
+  if ((r.visible && !want) || (r.culled && want)) {
+    if (++failures <= 10) std::printf("%s: quick says %s, the oracle %s\n", what, r.visible ? "visible" : "culled",
+                                      want ? "visible" : "culled");
+  }
+}
+
+// Runs `count` pairs of one kind and prints the share decided.
+template <class Make>
+double kind(const char* what, int count, Make&& make)
+{
+  const long d0 = decided, p0 = pairs;
+  float obb[16], vp[16];
+  for (int k = 0; k < count; ++k) {
+    make(obb, vp);
+    check(obb, vp, what);
+  }
+  const double share = static_cast<double>(decided - d0) / static_cast<double>(pairs - p0);
+  std::printf("%-28s %9d pairs, %.4f decided\n", what, count, share);
+  return share;
+}
+
+}  // namespace
+
+int main()
+{
+  // ordinary scenes: most pairs are decided, or the test would be no use
+  for (int ortho = 0; ortho < 2; ++ortho)
+    for (int reversed = 0; reversed < 2; ++reversed) {
+      const double share = kind(ortho ? "orthographic" : "perspective", 400000, [&](float* o, float* vp) {
+        view_projection(vp, ortho, reversed);
+        object(o, 1000, 2);
+      });
+      if (share < (reversed ? 0.9 : 0.97)) {
+        std::printf("only %.4f decided\n", share);
+        ++failures;
+      }
+    }
+  // large boxes near the eye: corners on both sides of several planes, w of both signs
+  kind("large boxes", 400000, [](float* o, float* vp) {
+    view_projection(vp, pick(3) == 0, pick(4) == 0);
+    object(o, 100, uniform(1, 200));
+  });
+  // axis-aligned integer boxes against planes through integers: exact ties, where only the exact test counts
+  kind("ties", 400000, [](float* o, float* vp) {
+    for (int c = 0; c < 16; ++c) vp[c] = static_cast<float>(pick(3) - 1);
+    for (int c = 0; c < 16; ++c) o[c] = c % 4 == 3 ? (c == 3 ? 1.0f : 0.0f) : static_cast<float>(pick(7) - 3);
+  });
+  // boxes whose nearest corner lies within a few rounding errors of a plane
+  kind("grazing", 800000, [](float* o, float* vp) {
+    view_projection(vp, false, false);
+    object(o, 500, 2);
+    const int axis = pick(3);
+    const double sign = pick(2) ? 1 : -1;
+    double n[4];
+    for (int j = 0; j < 4; ++j) n[j] = vp[4 * j + 3] + sign * vp[4 * j + axis];
+    const double len2 = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
+    if (len2 == 0) return;
+    double far = -1e300, d = n[3];
+    for (int c = 0; c < 3; ++c) d += n[c] * o[c];
+    far = d;
+    for (int e = 1; e < 4; ++e) {
+      double t = 0;
+      for (int c = 0; c < 3; ++c) t += n[c] * o[4 * e + c];
+      if (t > 0) far += t;
+    }
+    const double move = -far / len2 * (1 + uniform(-2, 2) * 0x1p-22);
+    for (int c = 0; c < 3; ++c) o[c] = static_cast<float>(o[c] + move * n[c]);
+  });
+  // every magnitude: scenes scaled by powers of two, down to denormals and up to overflow
+  kind("scaled", 800000, [](float* o, float* vp) {
+    view_projection(vp, pick(2), false);
+    object(o, 1000, 2);
+    const int so = pick(260) - 130, sv = pick(260) - 130;
+    for (int c = 0; c < 16; ++c)
+      if (c % 4 != 3) o[c] = std::ldexp(o[c], so);
+    if (pick(2)) o[3] = std::ldexp(1.0f, pick(260) - 130);
+    for (int c = 0; c < 16; ++c) vp[c] = std::ldexp(vp[c], sv + (pick(4) ? 0 : pick(40) - 20));
+  });
+  // every element scaled by itself
+  kind("wild", 800000, [](float* o, float* vp) {
+    view_projection(vp, pick(2), false);
+    object(o, 1000, 2);
+    for (int c = 0; c < 16; ++c) {
+      if (pick(3) == 0) o[c] = std::ldexp(o[c], pick(200) - 100);
+      if (pick(3) == 0) vp[c] = std::ldexp(vp[c], pick(200) - 100);
+    }
+  });
+  // zeros, denormals, limits, infinities and NaN in any place
+  kind("odd values", 800000, [](float* o, float* vp) {
+    view_projection(vp, pick(2), false);
+    object(o, 1000, 2);
+    const int n = 1 + pick(4), odd = static_cast<int>(sizeof kOdd / sizeof kOdd[0]);
+    for (int k = 0; k < n; ++k) (pick(2) ? o : vp)[pick(16)] = kOdd[pick(odd)];
+  });
+  // projective object matrices: edges with a w component
+  kind("projective objects", 400000, [](float* o, float* vp) {
+    view_projection(vp, pick(2), false);
+    object(o, 100, 20);
+    for (int e = 0; e < 4; ++e)
+      if (pick(2)) o[4 * e + 3] = static_cast<float>(uniform(-2, 2));
+  });
+  std::printf("quick cull: %ld of %ld pairs decided\nquick cull: %ld failures\n", decided, pairs, failures);
+  return failures ? 1 : 0;
+}

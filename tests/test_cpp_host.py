@@ -34,6 +34,14 @@ def test_tree_plan_tiles_emulated():
     assert "tree plan: 0 failures" in out
 
 
+def test_quick_cull_decides_as_the_oracle():
+    """Whatever the quick visibility test (quick_cull.hpp) decides is the oracle's
+    answer: ordinary scenes, grazing boxes and ties, every magnitude, infinities
+    and NaN, projective matrices."""
+    out = run("quick_cull_test")
+    assert "quick cull: 0 failures" in out
+
+
 @pytest.mark.gpu
 def test_gpu_tree_matches_reference_trace():
     out = run("tree_gpu_test", str(GOLDEN / "ref_tree_trace.bin"))
