@@ -179,7 +179,7 @@ typedef struct dpc_batch_config {
   uint32_t objects_per_lane; /* 1, 2 or 4: a wave owns 64*objects_per_lane objects */
   uint32_t block_threads;    /* 64, 128, 256 */
   uint32_t waves_per_cu;     /* persistent grid size = CUs * waves_per_cu / waves per block */
-  uint32_t max_frusta_per_item; /* split a tile's frustum list into chunks of this size (0 = no split) */
+  uint32_t max_frusta_per_item; /* split a tile's frustum list into chunks of this size (0 = the plan chooses) */
 } dpc_batch_config;
 
 typedef struct dpc_batch_plan dpc_batch_plan;

@@ -15,7 +15,7 @@
 //
 // What bounds it: with many frusta per object, vector instructions: 60 per
 // frustum and 64 objects with the quick test (55 with two objects per lane), 190
-// when each pair took the exact test.  500,003 objects x 32 frusta, two objects per lane: 109 -> 47 us;
+// when each pair took the exact test.  500,003 objects x 32 frusta: 109 -> 36 us;
 // 64 frusta over 64 groups of 2,097,152 objects: 40 -> 36 us, 4.5 TB/s, now bound
 // by reading the objects.
 //
@@ -453,7 +453,7 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   *out = nullptr;
   if ((n_groups && !groups) || (n_pairs && !pairs))
     return set_error(DPC_ERR_INVALID_ARGUMENT, "dpc_batch_plan_create: null groups/pairs");
-  dpc_batch_config c{2, 256, 8, 0};
+  dpc_batch_config c{1, 256, 24, 0};
   if (cfg) c = *cfg;
   int rc = validate_config(c);
   if (rc) return rc;
@@ -470,6 +470,7 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   plan->cfg = c;
   plan->n_frusta = n_frusta;
   (void)hipGetDevice(&plan->device);
+  const uint64_t cus = static_cast<uint64_t>(std::max(device_cu_count(), 1));
 
   // Pairs grouped by group, frusta ascending within a group.
   std::vector<uint32_t> order(n_pairs);
@@ -487,12 +488,45 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   }
   for (size_t g = 0; g < n_groups; ++g) group_pair_begin[g + 1] += group_pair_begin[g];
 
+  if (!cfg) {
+    // Two objects per lane halve the per-frustum work that a wave does once for all
+    // its objects, and halve the waves: worth it where both are plenty (300,000
+    // objects x 32 views: 25.5 us against 26.7 with one; 1,000,000 x 8: 27.3
+    // against 26.1; 150,000 objects, 13,000 (tile, view) pairs: 10.0 against 8.7).
+    uint64_t tiles = 0, tile_pairs = 0;
+    for (size_t g = 0; g < n_groups; ++g) {
+      const uint64_t n = group_pair_begin[g + 1] - group_pair_begin[g], t = (groups[g].count + kWave - 1) / kWave;
+      tiles += n ? t : 0;
+      tile_pairs += n * t;
+    }
+    if (tiles >= 16ull * cus && tile_pairs >= 16 * tiles) plan->cfg.objects_per_lane = c.objects_per_lane = 2;
+  }
   const uint64_t tile_objects = static_cast<uint64_t>(kWave) * c.objects_per_lane;
+  if (c.max_frusta_per_item == 0) {
+    // Where the tiles alone would leave the device idle, lists are split into
+    // slices of a length that gives about ten work items per CU (79 tiles x 64
+    // views: 15 us unsplit, 5.6 us in slices of 2, 5.9 of 1, 6.0 of 4; 625 tiles x
+    // 13 views: 6.6 us in slices of 4, 6.9 of 2, 7.4 of 8).  With eight tiles per
+    // CU a slice's second read of the objects costs more than it gives (2,344
+    // tiles x 6 views: 8.7 us unsplit, 9.9 in slices of 3); lists are then cut only
+    // after 16 views, so that the last items of a long launch are short (4,688
+    // tiles x 32 views: 25.5 us, 27 unsplit).
+    uint64_t tiles = 0, tile_pairs = 0;
+    for (size_t g = 0; g < n_groups; ++g) {
+      const uint64_t n = group_pair_begin[g + 1] - group_pair_begin[g];
+      const uint64_t t = (groups[g].count + tile_objects - 1) / tile_objects;
+      tiles += n ? t : 0;
+      tile_pairs += n * t;
+    }
+    c.max_frusta_per_item =
+        tiles >= 8 * cus ? 16u : static_cast<uint32_t>(std::clamp<uint64_t>(tile_pairs / (10 * cus), 1, 16));
+  }
   std::vector<WorkItem> items;
   for (size_t g = 0; g < n_groups; ++g) {
     const uint64_t pb = group_pair_begin[g], pe = group_pair_begin[g + 1];
     if (pb == pe || groups[g].count == 0) continue;
-    const uint64_t chunk = c.max_frusta_per_item ? c.max_frusta_per_item : (pe - pb);
+    const uint64_t slices = (pe - pb + c.max_frusta_per_item - 1) / c.max_frusta_per_item;
+    const uint64_t chunk = (pe - pb + slices - 1) / slices;
     for (uint64_t t0 = 0; t0 < groups[g].count; t0 += tile_objects) {
       const uint32_t cnt = static_cast<uint32_t>(std::min<uint64_t>(tile_objects, groups[g].count - t0));
       for (uint64_t q = pb; q < pe; q += chunk) {
