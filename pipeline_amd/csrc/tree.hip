@@ -220,6 +220,7 @@ __global__ __launch_bounds__(kSmallThreads) void tree_small_levels_kernel(const 
 // written to memory once per step, after its pieces.
 using tileplan::Seg;
 constexpr uint32_t kMaxSegs = 64;
+static_assert(kMaxSegs == kWave, "one lane per piece");
 constexpr uint32_t kNoSeg = 0xFFFFFFFFu;
 
 struct StepIn {
@@ -339,41 +340,48 @@ __device__ __forceinline__ float4 pick_row(const StepIn& in)
 // Computes the pieces [a, b) of one step.  Each thread has at most one slot in
 // the step: its rows go to the ring (kept passes) inside the loop, and to
 // memory (when the tile owns the slot and it changed) after the loop.
+//
+// What bounds it: the pieces of a tile's top passes follow each other in one
+// wave, so each piece's instructions are latency on the tile's critical path.
+// Everything that does not depend on the parent's rows (the thread's piece, ring
+// positions, its row of the local matrix) is therefore worked out before the
+// loop, once for all pieces; a piece is then one round of LDS reads, the
+// product, and the writes.  barriers: bit j set = an LDS barrier follows piece j.
 template <bool HasDirty, unsigned MaxRing>
-__device__ __forceinline__ void run_step(const StepIn& in, const Seg* sg, uint32_t a, uint32_t b, uint32_t ring_len,
-                                         const float4* W, size_t ld, const uint8_t* dirty_world,
-                                         const __amdgpu_buffer_rsrc_t (&rw)[4], __amdgpu_buffer_rsrc_t rdw,
-                                         float4 (&rows)[4][MaxRing], uint8_t (&flag)[MaxRing])
+__device__ __forceinline__ void run_step(const StepIn& in, const Seg* sg, uint32_t a, uint32_t b,
+                                         unsigned long long barriers, uint32_t ring_len, const float4* W, size_t ld,
+                                         const uint8_t* dirty_world, const __amdgpu_buffer_rsrc_t (&rw)[4],
+                                         __amdgpu_buffer_rsrc_t rdw, float4 (&rows)[4][MaxRing],
+                                         uint8_t (&flag)[MaxRing])
 {
-  bool store = false, quad = false;
+  // the thread's piece (an idle thread reads some piece and takes part in none)
+  const Seg* const mine = &sg[in.seg != kNoSeg ? in.seg : 0u];
+  const uint4 h = *reinterpret_cast<const uint4*>(mine);
+  const uint2 pr = *reinterpret_cast<const uint2*>(&mine->pfirst);  // pfirst, pcount | pring << 16
+  const uint32_t first = h.x, ring = h.z & 0xFFFFu, flags = h.z >> 16, own_end = h.w;
+  const uint64_t p = in.p;
+  const bool valid = p < ld;  // a parent outside the arrays is never read (as in propagate_slot)
+  const uint32_t d = static_cast<uint32_t>(p) - pr.x;
+  const bool staged = valid && !(flags & tileplan::kFromMemory) && d < (pr.y & 0xFFFFu);
+  uint32_t i = (pr.y >> 16) + d;  // the parent's ring position
+  i = i >= ring_len ? i - ring_len : i;
+  i = staged && i < MaxRing ? i : 0u;
+  uint32_t o = ring + (in.slot - first);  // the slot's own
+  o = o >= ring_len ? o - ring_len : o;
+  o = o < MaxRing ? o : 0u;  // the plan keeps positions below its ring length (at most MaxRing)
+  const bool quad = (flags & tileplan::kQuad) != 0, keep = (flags & tileplan::kStaged) != 0;
+  float4 l0 = in.l0;
+  if (__builtin_amdgcn_ballot_w64(quad) != 0) l0 = quad ? pick_row(in) : l0;  // this thread's row only
+  bool store = false;
   float4 w0 = make_float4(0.f, 0.f, 0.f, 0.f), w1 = w0, w2 = w0, w3 = w0;
-  // a < b <= n for every step of a valid plan; b <= n always (load_step)
-  const uint32_t a0 = a < b ? a : 0u;
-  SegHead h = seg_head(sg, a0);
-  uint2 pr = *reinterpret_cast<const uint2*>(&sg[a0].pfirst);  // the parent range: pfirst, pcount | pring << 16
   for (uint32_t j = a; j < b; ++j) {
-    // the next piece's descriptor (both halves), read while this one is computed
-    const uint32_t jn = j + 1 < b ? j + 1 : j;
-    const uint4 hn = *reinterpret_cast<const uint4*>(&sg[jn]);
-    const uint2 prn = *reinterpret_cast<const uint2*>(&sg[jn].pfirst);
     if (in.seg == j) {
-      const uint32_t pfirst = __builtin_amdgcn_readfirstlane(pr.x);
-      const uint32_t pp = __builtin_amdgcn_readfirstlane(pr.y);
-      const uint32_t pcount = pp & 0xFFFFu, pring = pp >> 16;
-      const uint64_t p = in.p;
-      const bool valid = p < ld;  // a parent outside the arrays is never read (as in propagate_slot)
-      const uint32_t d = static_cast<uint32_t>(p) - pfirst;
-      const bool staged = valid && !(h.flags & tileplan::kFromMemory) && d < pcount;
-      uint32_t i = pring + d;
-      i = i >= ring_len ? i - ring_len : i;
-      i = staged && i < MaxRing ? i : 0u;
       // the flag and the rows in one round of LDS loads (the rows are used
       // only when the flag says the parent was recomputed)
       const uint32_t f = flag[i];
       float4 p0 = rows[0][i], p1 = rows[1][i], p2 = rows[2][i], p3 = rows[3][i];
-      const uint32_t dp_lds = staged ? f : 0u;
       bool dirty = false;
-      if (dp_lds) {  // the parent was recomputed by this tile: its rows are in the ring
+      if (staged && f) {  // the parent was recomputed by this tile: its rows are in the ring
         dirty = true;
       } else if (valid && (!staged || in.dl)) {
         const uint32_t pu = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
@@ -398,46 +406,39 @@ __device__ __forceinline__ void run_step(const StepIn& in, const Seg* sg, uint32
           dirty = (in.dl | (staged ? 0u : dp)) != 0;
         }
       }
-      quad = (h.flags & tileplan::kQuad) != 0;
       if (dirty) {
-        if (quad) {  // this thread's row only: a quarter of the arithmetic latency
-          w0 = rowmat(pick_row(in), p0, p1, p2, p3);
-          w1 = w0;
-          w2 = w0;
-          w3 = w0;
+        // (a piece's threads are all of one kind: a scalar branch, which keeps the
+        // other three rows' arithmetic off the one-row path)
+        if (__builtin_amdgcn_ballot_w64(quad) != 0) {
+          w0 = rowmat(l0, p0, p1, p2, p3);  // one row per thread: a quarter of the arithmetic latency
+          if (keep) rows[in.row][o] = w0;
         } else {
           w0 = rowmat(in.l0, p0, p1, p2, p3);
           w1 = rowmat(in.l1, p0, p1, p2, p3);
           w2 = rowmat(in.l2, p0, p1, p2, p3);
           w3 = rowmat(in.l3, p0, p1, p2, p3);
+          if (keep) {
+            rows[0][o] = w0;
+            rows[1][o] = w1;
+            rows[2][o] = w2;
+            rows[3][o] = w3;
+          }
         }
       }
-      if (h.flags & tileplan::kStaged) {
-        uint32_t o = h.ring + (in.slot - h.first);
-        o = o >= ring_len ? o - ring_len : o;
-        o = o < MaxRing ? o : 0u;  // the plan keeps positions below its ring length (at most MaxRing)
-        if (dirty) {
-          if (!quad || in.row == 0) rows[0][o] = w0;
-          if (!quad || in.row == 1) rows[1][o] = w1;
-          if (!quad || in.row == 2) rows[2][o] = w2;
-          if (!quad || in.row == 3) rows[3][o] = w3;
-        }
-        flag[o] = dirty ? 1 : 0;
-      }
-      store = dirty && in.slot < h.own_end;
+      if (keep) flag[o] = dirty ? 1 : 0;
+      store = dirty && in.slot < own_end;
     }
     // passes written and read within one wave need no barrier: a wave's LDS
     // operations execute in order
-    if (h.flags & tileplan::kBarrier) lds_barrier();
-    h = decode_head(hn);
-    pr = prn;
+    if ((barriers >> j) & 1) lds_barrier();
   }
   // one row plane per thread of a kQuad slot, all four otherwise
   const uint32_t off = store ? in.slot * 16u : kNoStore;
-  store_row(w0, rw[0], !quad || in.row == 0 ? off : kNoStore);
-  store_row(w1, rw[1], !quad || in.row == 1 ? off : kNoStore);
-  store_row(w2, rw[2], !quad || in.row == 2 ? off : kNoStore);
-  store_row(w3, rw[3], !quad || in.row == 3 ? off : kNoStore);
+  const bool all = store && !quad;
+  store_row(w0, rw[0], store && in.row == 0 ? off : kNoStore);
+  store_row(quad ? w0 : w1, rw[1], all || (store && in.row == 1) ? off : kNoStore);
+  store_row(quad ? w0 : w2, rw[2], all || (store && in.row == 2) ? off : kNoStore);
+  store_row(quad ? w0 : w3, rw[3], all || (store && in.row == 3) ? off : kNoStore);
   __builtin_amdgcn_raw_buffer_store_b8(static_cast<unsigned char>(1), rdw, store && in.row == 0 ? in.slot : kNoStore,
                                        0, 0);
   // the step's loaded registers are consumed on every path: reusing them for a
@@ -472,6 +473,9 @@ __global__ __launch_bounds__(Threads) void tree_tile_kernel(const float4* __rest
   const uint32_t n = min(__builtin_amdgcn_readfirstlane(sg[0].tile_pieces), kMaxSegs);
   const uint32_t steps = min(__builtin_amdgcn_readfirstlane(sg[0].tile_steps), n);
   if (n == 0) return;  // (the plan gives every tile at least one piece)
+  // pieces that an LDS barrier follows (kMaxSegs pieces: one bit per lane)
+  const unsigned long long barriers = __builtin_amdgcn_ballot_w64(
+      (sg[threadIdx.x & (kWave - 1)].flags & tileplan::kBarrier) != 0);
   const uint32_t rec = static_cast<uint32_t>(ld * 16);  // ld <= kMaxBufferSlots (checked by the plan)
   const __amdgpu_buffer_rsrc_t rw[4] = {__builtin_amdgcn_make_buffer_rsrc(W, 0, rec, kRawBufferDword3),
                                         __builtin_amdgcn_make_buffer_rsrc(W + ld, 0, rec, kRawBufferDword3),
@@ -492,17 +496,17 @@ __global__ __launch_bounds__(Threads) void tree_tile_kernel(const float4* __rest
   uint32_t k = 0;
   for (; k + 2 < steps; k += 3) {
     const uint32_t pd = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pc, C);
-    run_step<HasDirty, MaxRing>(A, sg, pa, pb, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+    run_step<HasDirty, MaxRing>(A, sg, pa, pb, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
     const uint32_t pe = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pd < n ? pd : pc, A);
-    run_step<HasDirty, MaxRing>(B, sg, pb, pc, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+    run_step<HasDirty, MaxRing>(B, sg, pb, pc, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
     const uint32_t pf = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pe < n ? pe : pc, B);
-    run_step<HasDirty, MaxRing>(C, sg, pc, pd, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+    run_step<HasDirty, MaxRing>(C, sg, pc, pd, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
     pa = pd;
     pb = pe;
     pc = pf;
   }
-  if (k < steps) run_step<HasDirty, MaxRing>(A, sg, pa, pb, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
-  if (k + 1 < steps) run_step<HasDirty, MaxRing>(B, sg, pb, pc, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+  if (k < steps) run_step<HasDirty, MaxRing>(A, sg, pa, pb, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+  if (k + 1 < steps) run_step<HasDirty, MaxRing>(B, sg, pb, pc, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
 }
 
 // dp::math::invertTranspose (dp/math/Matmnt.h:1171-1201) of W[s]: 2x2 minors of
