@@ -610,7 +610,13 @@ struct dpc_tree_plan {
 
 namespace {
 
-constexpr uint32_t kDefaultTileThreads = 1024;  // measured fastest on the 1M-node tree (27.5 us vs 29.3 at 512)
+// Threads of a tile workgroup where the caller leaves them to the plan.  Smaller
+// workgroups split a tree over more CUs, shorten each tile's steps and mix the
+// reads of one tile with the writes of another; larger ones recompute fewer
+// shared ancestors.  Full propagation with 256 / 512 / 1024 threads: 3,000 nodes
+// 6.6 / 6.5 / 7.3 us, 50,000 8.1 / 9.1 / 9.5, 250,007 13.9 / 12.9 / 12.8, 500,000
+// 16.7 / 16.1 / 16.9, 700,000 25.6 / 25.6 / 30.9, 1,000,000 35.4 / 37.4 / 37.3.
+uint32_t default_tile_threads(uint64_t slots) { return slots > 150000 && slots < 600000 ? 512 : 256; }
 constexpr size_t kMaxRunPasses = 32;
 
 template <bool HasDirty>
@@ -734,13 +740,13 @@ int dpc_tree_plan_create(const uint32_t* h_parent_slot, size_t ld, const uint64_
     // (Tree::compute visits no level and notifies an empty change set)
     auto plan = std::make_unique<dpc_tree_plan>();
     plan->ld = ld;
-    plan->threads = tile_slots ? tile_slots : kDefaultTileThreads;
+    plan->threads = tile_slots ? tile_slots : default_tile_threads(h_level_offsets[n_levels]);
     *out = plan.release();
     return DPC_OK;
   }
   auto plan = std::make_unique<dpc_tree_plan>();
   plan->ld = ld;
-  plan->threads = tile_slots ? tile_slots : kDefaultTileThreads;
+  plan->threads = tile_slots ? tile_slots : default_tile_threads(h_level_offsets[n_levels]);
   const uint32_t max_ring = tile_max_ring(plan->threads);
   // workgroups the device holds at once: CUs x tile workgroups per CU
   int dev = 0, cus = 0, per_cu = 0;
