@@ -99,14 +99,6 @@ struct Queue {
   QueueWord word[kCapacity];
 };
 
-// Orders a wave's LDS accesses across its lanes (they execute in order; the
-// compiler must not move them).
-__device__ __forceinline__ void wave_lds_order()
-{
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // The exact test of the queue's n entries, then the stores of its n_words words.
 template <int K>
 __device__ __forceinline__ void drain(Queue<K>& queue, uint32_t n, uint32_t n_words, uint32_t lane,

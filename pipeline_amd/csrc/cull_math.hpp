@@ -30,6 +30,14 @@ __device__ __forceinline__ void lds_barrier()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders a wave's LDS accesses across its lanes (they execute in order; the
+// compiler must not move them).
+__device__ __forceinline__ void wave_lds_order()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // A 4x4 row-major matrix passed by value in kernel arguments: the compiler
 // loads it into scalar registers once per wave, and the VALU multiplies read
 // it from there.

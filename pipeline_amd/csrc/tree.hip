@@ -569,14 +569,80 @@ __global__ __launch_bounds__(kTreeThreads) void inverse_transpose_kernel(const f
   if (ok) ok[s] = good ? 1 : 0;
 }
 
-__global__ void bytes_to_bits_kernel(const uint8_t* __restrict__ bytes, const uint32_t* __restrict__ index_of_slot,
-                                     size_t n, uint32_t* __restrict__ bits, size_t n_bits)
+// One bit per set byte.  A wave takes kBitsSlots consecutive slots and gathers
+// their bits in LDS, in a window of kBitsWindow bits from its lowest slot's index
+// on; each word that holds a bit goes to memory with one atomic.  What lies outside
+// gets a second window, and what lies outside that goes to memory bit by bit.
+// Slots are level-major and a level's indices ascend, so a wave's indices lie
+// close together (within a few of each other among leaves), in two places where a
+// level ends: a word then takes about one atomic per level instead of one per
+// slot.  What bounds it is those atomics: words are shared by waves on different
+// XCDs, whose L2s pass them to and fro, and a wave's atomics to one word follow
+// each other.  One atomic per set byte took 33.7 us for 700,000 set bytes and 9.9
+// us for 21,000 of 250,007; this takes 7.4 and 5.2.
+constexpr unsigned kBitsPerLane = 8;
+constexpr unsigned kBitsSlots = kWave * kBitsPerLane;
+constexpr unsigned kBitsWindow = 8192;
+static_assert(kBitsWindow == kWave * 4 * 32, "four window words per lane");
+
+__global__ __launch_bounds__(kTreeThreads) void bytes_to_bits_kernel(const uint8_t* __restrict__ bytes,
+                                                                     const uint32_t* __restrict__ index_of_slot,
+                                                                     size_t n, uint32_t* __restrict__ bits,
+                                                                     size_t n_bits)
 {
-  const size_t s = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (s >= n || bytes[s] == 0) return;
-  const size_t i = index_of_slot ? static_cast<size_t>(index_of_slot[s]) : s;
-  if (i >= n_bits) return;
-  atomicOr(&bits[i >> 5], 1u << (i & 31));
+  __shared__ uint4 windows[kTreeThreads / kWave][kWave];
+  const unsigned lane = threadIdx.x & (kWave - 1);
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const size_t first = (static_cast<size_t>(blockIdx.x) * (kTreeThreads / kWave) + wave) * kBitsSlots;
+  if (first >= n) return;
+  uint32_t* const window = reinterpret_cast<uint32_t*>(windows[wave]);
+  bool left[kBitsPerLane];  // bits not yet written
+#pragma unroll
+  for (unsigned k = 0; k < kBitsPerLane; ++k) {  // (clamped: every load is issued before any is waited for)
+    const size_t s = first + k * kWave + lane;
+    left[k] = bytes[s < n ? s : n - 1] != 0 && s < n;
+  }
+  size_t index[kBitsPerLane];
+#pragma unroll
+  for (unsigned k = 0; k < kBitsPerLane; ++k) {
+    const size_t s = first + k * kWave + lane;
+    index[k] = left[k] ? (index_of_slot ? static_cast<size_t>(index_of_slot[s]) : s) : n_bits;
+    left[k] = index[k] < n_bits;
+  }
+  for (int pass = 0; pass < 2; ++pass) {
+    // the wave's first unwritten slot (the lowest index, where indices ascend)
+    size_t base = ~size_t(0);
+#pragma unroll
+    for (unsigned k = kBitsPerLane; k-- > 0;) {
+      const unsigned long long m = ballot(left[k]);
+      if (m == 0) continue;
+      const int from = __builtin_ctzll(m);
+      base = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(index[k]), from)) |
+             static_cast<size_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(index[k] >> 32), from))) << 32;
+    }
+    if (base == ~size_t(0)) return;
+    base &= ~size_t(31);
+    windows[wave][lane] = make_uint4(0u, 0u, 0u, 0u);
+    wave_lds_order();
+#pragma unroll
+    for (unsigned k = 0; k < kBitsPerLane; ++k) {
+      const size_t at = index[k] - base;  // (an index below the base wraps to a large value)
+      if (left[k] && at < kBitsWindow) {
+        atomicOr(&window[at >> 5], 1u << (at & 31));
+        left[k] = false;
+      }
+    }
+    wave_lds_order();
+#pragma unroll
+    for (unsigned w = 0; w < 4; ++w) {  // consecutive lanes take consecutive words
+      const uint32_t v = window[w * kWave + lane];
+      if (v) atomicOr(&bits[(base >> 5) + w * kWave + lane], v);
+    }
+    wave_lds_order();
+  }
+#pragma unroll
+  for (unsigned k = 0; k < kBitsPerLane; ++k)
+    if (left[k]) atomicOr(&bits[index[k] >> 5], 1u << (index[k] & 31));
 }
 
 }  // namespace
@@ -716,8 +782,9 @@ int dpc_bytes_to_bits_indexed(const uint8_t* d_bytes, const uint32_t* d_index_of
 {
   if (n_slots == 0 || n_bits == 0) return DPC_OK;
   if (!d_bytes || !d_bits) return set_error(DPC_ERR_INVALID_ARGUMENT, "dpc_bytes_to_bits_indexed: null pointer");
-  hipLaunchKernelGGL(bytes_to_bits_kernel, dim3(static_cast<unsigned>((n_slots + 255) / 256)), dim3(256), 0,
-                     as_stream(stream), d_bytes, d_index_of_slot, n_slots, d_bits, n_bits);
+  constexpr size_t per_block = kBitsSlots * (kTreeThreads / kWave);
+  hipLaunchKernelGGL(bytes_to_bits_kernel, dim3(static_cast<unsigned>((n_slots + per_block - 1) / per_block)),
+                     dim3(kTreeThreads), 0, as_stream(stream), d_bytes, d_index_of_slot, n_slots, d_bits, n_bits);
   return check_launch("bytes_to_bits_kernel");
 }
 
