@@ -565,33 +565,43 @@ __device__ __forceinline__ unsigned long long diff_word_clamped(const unsigned l
   return w < n_words ? (x & keep) : 0ull;
 }
 
-// Exclusive scan over a block of Threads threads (lds: Threads / 64 + 1 words).
-template <unsigned Threads = kDiffThreads>
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* lds, uint32_t* total)
+// Inclusive scan over a wave (data-parallel primitives: within rows of 16 lanes,
+// then the last lane of each half row pair, then of the lower half).
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v)
 {
-  // Wave-level inclusive scan, then scan of the wave totals.
-  const unsigned lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  uint32_t x = v;
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t y = __shfl_up(x, off, kWave);
-    if (lane >= static_cast<unsigned>(off)) x += y;
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xa, 0xf, true);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xc, 0xf, true);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Position of this thread's first of `count` entries: every thread's `before`
+// together, and the counts of the threads before it; *total: all of both.  One
+// barrier: each wave leaves its two sums in LDS (lds: 2 * Threads / 64 words) and
+// adds up all waves' itself.
+template <unsigned Threads>
+__device__ __forceinline__ uint32_t block_position(uint32_t count, uint32_t before, uint32_t* lds, uint32_t* total)
+{
+  constexpr unsigned kWaves = Threads / kWave;
+  static_assert(kWaves <= 16, "one row of lanes holds the waves' sums");
+  const unsigned lane = threadIdx.x & (kWave - 1);
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t scan = wave_inclusive_scan(count);
+  const uint32_t sum = wave_inclusive_scan(before);
+  if (lane == kWave - 1) {
+    lds[wave] = scan;
+    lds[kWaves + wave] = sum;
   }
-  if (lane == kWave - 1) lds[wave] = x;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t run = 0;
-    for (unsigned k = 0; k < Threads / kWave; ++k) {
-      const uint32_t t = lds[k];
-      lds[k] = run;
-      run += t;
-    }
-    lds[Threads / kWave] = run;
-  }
-  __syncthreads();
-  const uint32_t r = lds[wave] + x - v;
-  *total = lds[Threads / kWave];
-  __syncthreads();
-  return r;
+  lds_barrier();
+  const uint32_t c = lane < kWaves ? lds[lane] : 0u;
+  const uint32_t b = lane < kWaves ? lds[kWaves + lane] : 0u;
+  const uint32_t to_here = wave_inclusive_scan(b + (lane < wave ? c : 0u));
+  const uint32_t all = wave_inclusive_scan(b + c);
+  *total = __builtin_amdgcn_readlane(static_cast<int>(all), kWave - 1);
+  return __builtin_amdgcn_readlane(static_cast<int>(to_here), kWave - 1) + scan - count;
 }
 
 __global__ __launch_bounds__(kDiffThreads) void diff_count_kernel(const unsigned long long* __restrict__ old_w,
@@ -599,11 +609,11 @@ __global__ __launch_bounds__(kDiffThreads) void diff_count_kernel(const unsigned
                                                                   size_t n_words, size_t n_bits,
                                                                   uint32_t* __restrict__ block_count)
 {
-  __shared__ uint32_t lds[kDiffThreads / kWave + 1];
+  __shared__ uint32_t lds[2 * kDiffThreads / kWave];
   const size_t w = static_cast<size_t>(blockIdx.x) * kDiffThreads + threadIdx.x;
   const uint32_t c = __popcll(diff_word(old_w, new_w, w, n_words, n_bits));
   uint32_t total;
-  block_exclusive_scan(c, lds, &total);
+  block_position<kDiffThreads>(c, 0u, lds, &total);
   if (threadIdx.x == 0) block_count[blockIdx.x] = total;
 }
 
@@ -611,15 +621,16 @@ __global__ __launch_bounds__(kDiffThreads) void diff_count_kernel(const unsigned
 __global__ __launch_bounds__(kDiffThreads) void diff_scan_kernel(uint32_t* __restrict__ block_count, size_t n_blocks,
                                                                  uint32_t* __restrict__ d_count)
 {
-  __shared__ uint32_t lds[kDiffThreads / kWave + 1];
+  __shared__ uint32_t lds[2 * kDiffThreads / kWave];
   uint32_t carry = 0;
   for (size_t base = 0; base < n_blocks; base += kDiffThreads) {
     const size_t k = base + threadIdx.x;
     const uint32_t v = k < n_blocks ? block_count[k] : 0u;
     uint32_t total;
-    const uint32_t ex = block_exclusive_scan(v, lds, &total);
+    const uint32_t ex = block_position<kDiffThreads>(v, 0u, lds, &total);
     if (k < n_blocks) block_count[k] = carry + ex;
     carry += total;
+    lds_barrier();  // (the next round overwrites what this one has read)
   }
   if (threadIdx.x == 0) *d_count = carry;
 }
@@ -630,11 +641,11 @@ __global__ __launch_bounds__(kDiffThreads) void diff_write_kernel(unsigned long 
                                                                   const uint32_t* __restrict__ block_offset,
                                                                   uint32_t* __restrict__ out, int update_old)
 {
-  __shared__ uint32_t lds[kDiffThreads / kWave + 1];
+  __shared__ uint32_t lds[2 * kDiffThreads / kWave];
   const size_t w = static_cast<size_t>(blockIdx.x) * kDiffThreads + threadIdx.x;
   unsigned long long x = diff_word(old_w, new_w, w, n_words, n_bits);
   uint32_t total;
-  uint32_t pos = block_offset[blockIdx.x] + block_exclusive_scan(__popcll(x), lds, &total);
+  uint32_t pos = block_offset[blockIdx.x] + block_position<kDiffThreads>(__popcll(x), 0u, lds, &total);
   while (x) {
     const unsigned b = __ffsll(static_cast<long long>(x)) - 1;
     out[pos++] = static_cast<uint32_t>(w * 64 + b);
@@ -655,7 +666,7 @@ __global__ __launch_bounds__(kDiffThreads) void diff_write_direct_kernel(unsigne
                                                                          uint32_t* __restrict__ out, int update_old,
                                                                          uint32_t* __restrict__ d_count)
 {
-  __shared__ uint32_t lds[kDiffThreads / kWave + 1];
+  __shared__ uint32_t lds[2 * kDiffThreads / kWave];
   // this thread's words first: their loads are then in flight with those of the counts
   const size_t w = static_cast<size_t>(blockIdx.x) * kDiffThreads + threadIdx.x;
   unsigned long long new_bits;
@@ -671,11 +682,9 @@ __global__ __launch_bounds__(kDiffThreads) void diff_write_direct_kernel(unsigne
   uint32_t before = 0;
 #pragma unroll
   for (unsigned q = 0; q < kCountsPerThread; ++q) before += threadIdx.x + q * kDiffThreads < blockIdx.x ? v[q] : 0u;
-  uint32_t offset;
-  block_exclusive_scan(before, lds, &offset);
   uint32_t total;
-  uint32_t pos = offset + block_exclusive_scan(__popcll(x), lds, &total);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *d_count = offset + total;
+  uint32_t pos = block_position<kDiffThreads>(__popcll(x), before, lds, &total);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *d_count = total;
   while (x) {
     const unsigned b = __ffsll(static_cast<long long>(x)) - 1;
     out[pos++] = static_cast<uint32_t>(w * 64 + b);
@@ -702,7 +711,7 @@ __global__ __launch_bounds__(kDiffFusedThreads) void diff_write_fused_kernel(uns
                                                                              uint32_t* __restrict__ out, int update_old,
                                                                              uint32_t* __restrict__ d_count)
 {
-  __shared__ uint32_t lds[kDiffFusedThreads / kWave + 1];
+  __shared__ uint32_t lds[2 * kDiffFusedThreads / kWave];
   // this thread's words first: their loads are then in flight with those of the counts
   const size_t w = static_cast<size_t>(blockIdx.x) * kDiffFusedThreads + threadIdx.x;
   unsigned long long new_bits;
@@ -722,11 +731,9 @@ __global__ __launch_bounds__(kDiffFusedThreads) void diff_write_fused_kernel(uns
     const uint32_t part = byte_sum(c[q].w, byte_sum(c[q].z, byte_sum(c[q].y, byte_sum(c[q].x, 0u))));
     before += threadIdx.x + static_cast<size_t>(q) * kDiffFusedThreads < chunks ? part : 0u;
   }
-  uint32_t offset;
-  block_exclusive_scan<kDiffFusedThreads>(before, lds, &offset);
   uint32_t total;
-  uint32_t pos = offset + block_exclusive_scan<kDiffFusedThreads>(__popcll(x), lds, &total);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *d_count = offset + total;
+  uint32_t pos = block_position<kDiffFusedThreads>(__popcll(x), before, lds, &total);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *d_count = total;
   while (x) {
     const unsigned b = __ffsll(static_cast<long long>(x)) - 1;
     if (pos < n_bits) out[pos] = static_cast<uint32_t>(w * 64 + b);  // (always, when the counts match the masks)
