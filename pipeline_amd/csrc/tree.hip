@@ -232,67 +232,39 @@ struct StepIn {
   uint32_t row;   // the matrix row this thread computes in a kQuad piece (0 otherwise)
 };
 
-// A piece's fields as wave-uniform values (scalar registers): the first 16
-// bytes of a Seg in one LDS load, and the parent range in another.
-struct SegHead {
-  uint32_t first, count, pos, ring, flags, own_end;
+// What a wave keeps of its tile's pieces in registers: lane j holds piece j's
+// first thread; bit j of the masks says whether piece j ends its step, and whether
+// an LDS barrier follows it.
+struct Pieces {
+  uint32_t n;
+  uint32_t pos;
+  unsigned long long ends, barriers;
 };
 
-__device__ __forceinline__ SegHead decode_head(const uint4 h)
-{
-  SegHead r;
-  r.first = __builtin_amdgcn_readfirstlane(h.x);
-  const uint32_t cp = __builtin_amdgcn_readfirstlane(h.y);  // count | pos << 16
-  const uint32_t rf = __builtin_amdgcn_readfirstlane(h.z);  // ring | flags << 16
-  r.count = cp & 0xFFFFu;
-  r.pos = cp >> 16;
-  r.ring = rf & 0xFFFFu;
-  r.flags = rf >> 16;
-  r.own_end = __builtin_amdgcn_readfirstlane(h.w);
-  return r;
-}
-
-__device__ __forceinline__ SegHead seg_head(const Seg* sg, uint32_t j)
-{
-  return decode_head(*reinterpret_cast<const uint4*>(&sg[j]));
-}
-
-// Finds this thread's piece among the pieces of the step that starts at piece
-// g (four pieces per round of LDS loads) and issues its loads (unconditional
-// and clamped, as load_level).  Returns the first piece of the next step (n
-// when this is the last step).
+// Finds this thread's piece among the pieces of the step that starts at piece g,
+// the last whose first thread is not after it, and issues its loads
+// (unconditional and clamped, as load_level).  Returns the first piece of the next
+// step (n when this is the last step).  A step's pieces are compared from
+// registers, three instructions each: reading their descriptors from LDS in turn
+// took 0.8 us per step, twice before a tile's first loads.
 template <bool HasDirty>
 __device__ __forceinline__ uint32_t load_step(const float4* __restrict__ L, size_t ld,
                                               const uint32_t* __restrict__ parent,
-                                              const uint8_t* __restrict__ dirty_local, const Seg* sg, uint32_t n,
-                                              uint32_t g, StepIn& in)
+                                              const uint8_t* __restrict__ dirty_local, const Seg* sg,
+                                              const Pieces& pieces, uint32_t g, StepIn& in)
 {
-  uint32_t mine = kNoSeg, slot = 0, row = 0;
-  uint32_t next = g;
-  bool ended = false;
-  for (uint32_t j = g; !ended; j += 4) {
-    SegHead h[4];
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) h[q] = seg_head(sg, min(j + q, n - 1));
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {
-      if (ended) continue;
-      const uint32_t d = threadIdx.x - h[q].pos;
-      const uint32_t sh = (h[q].flags & tileplan::kQuad) ? 2u : 0u;  // threads per slot: 1 << sh
-      if (d < (h[q].count << sh)) {
-        mine = j + q;
-        slot = h[q].first + (d >> sh);
-        row = d & ((1u << sh) - 1u);
-      }
-      next = j + q + 1;
-      ended = (h[q].flags & tileplan::kStepEnd) || next >= n;
-    }
-  }
-  next = min(next, n);
-  in.seg = mine;
-  in.slot = slot;
-  in.row = row;
-  const uint64_t c = mine != kNoSeg ? slot : 0;
+  const uint32_t next = min(g + static_cast<uint32_t>(__builtin_ctzll(pieces.ends >> g)) + 1, pieces.n);
+  uint32_t mine = g;  // (a step's first piece starts at thread 0)
+  for (uint32_t j = g + 1; j < next; ++j)
+    mine += threadIdx.x >= static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(pieces.pos), static_cast<int>(j)));
+  const uint4 h = *reinterpret_cast<const uint4*>(&sg[mine]);  // first, count | pos << 16, ring | flags << 16
+  const uint32_t d = threadIdx.x - (h.y >> 16);
+  const uint32_t sh = (h.z >> 16) & tileplan::kQuad ? 2u : 0u;  // threads per slot: 1 << sh
+  const bool have = d < ((h.y & 0xFFFFu) << sh);
+  in.seg = have ? mine : kNoSeg;
+  in.slot = have ? h.x + (d >> sh) : 0u;
+  in.row = have ? d & ((1u << sh) - 1u) : 0u;
+  const uint64_t c = in.slot;
   in.p = parent[c];
   in.dl = HasDirty ? dirty_local[c] : 1u;
   in.l0 = L[c];
@@ -473,9 +445,14 @@ __global__ __launch_bounds__(Threads) void tree_tile_kernel(const float4* __rest
   const uint32_t n = min(__builtin_amdgcn_readfirstlane(sg[0].tile_pieces), kMaxSegs);
   const uint32_t steps = min(__builtin_amdgcn_readfirstlane(sg[0].tile_steps), n);
   if (n == 0) return;  // (the plan gives every tile at least one piece)
-  // pieces that an LDS barrier follows (kMaxSegs pieces: one bit per lane)
-  const unsigned long long barriers = __builtin_amdgcn_ballot_w64(
-      (sg[threadIdx.x & (kWave - 1)].flags & tileplan::kBarrier) != 0);
+  const unsigned lane = threadIdx.x & (kWave - 1);  // (kMaxSegs pieces: one per lane)
+  const uint32_t flags = sg[lane].flags;
+  Pieces pieces;
+  pieces.n = n;
+  pieces.pos = sg[lane].pos;
+  // (the tile's last piece ends a step: the marker bit is found from any piece of the tile)
+  pieces.ends = ballot((flags & tileplan::kStepEnd) != 0) | (1ull << (n - 1));
+  pieces.barriers = ballot((flags & tileplan::kBarrier) != 0);
   const uint32_t rec = static_cast<uint32_t>(ld * 16);  // ld <= kMaxBufferSlots (checked by the plan)
   const __amdgpu_buffer_rsrc_t rw[4] = {__builtin_amdgcn_make_buffer_rsrc(W, 0, rec, kRawBufferDword3),
                                         __builtin_amdgcn_make_buffer_rsrc(W + ld, 0, rec, kRawBufferDword3),
@@ -490,23 +467,25 @@ __global__ __launch_bounds__(Threads) void tree_tile_kernel(const float4* __rest
   // set consumed before the set is loaded again.  A load past the last step
   // repeats an earlier step's (unused).
   StepIn A, B, C;
-  uint32_t pa = 0;                                                                   // first piece of A's step
-  uint32_t pb = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pa, A);           // ... of B's
-  uint32_t pc = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pb < n ? pb : pa, B);  // ... of C's
+  uint32_t pa = 0;  // first piece of A's step, then of B's and C's
+  uint32_t pb = load_step<HasDirty>(L, ld, parent, dirty_local, sg, pieces, pa, A);
+  uint32_t pc = load_step<HasDirty>(L, ld, parent, dirty_local, sg, pieces, pb < n ? pb : pa, B);
   uint32_t k = 0;
   for (; k + 2 < steps; k += 3) {
-    const uint32_t pd = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pc, C);
-    run_step<HasDirty, MaxRing>(A, sg, pa, pb, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
-    const uint32_t pe = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pd < n ? pd : pc, A);
-    run_step<HasDirty, MaxRing>(B, sg, pb, pc, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
-    const uint32_t pf = load_step<HasDirty>(L, ld, parent, dirty_local, sg, n, pe < n ? pe : pc, B);
-    run_step<HasDirty, MaxRing>(C, sg, pc, pd, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+    const uint32_t pd = load_step<HasDirty>(L, ld, parent, dirty_local, sg, pieces, pc, C);
+    run_step<HasDirty, MaxRing>(A, sg, pa, pb, pieces.barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+    const uint32_t pe = load_step<HasDirty>(L, ld, parent, dirty_local, sg, pieces, pd < n ? pd : pc, A);
+    run_step<HasDirty, MaxRing>(B, sg, pb, pc, pieces.barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+    const uint32_t pf = load_step<HasDirty>(L, ld, parent, dirty_local, sg, pieces, pe < n ? pe : pc, B);
+    run_step<HasDirty, MaxRing>(C, sg, pc, pd, pieces.barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
     pa = pd;
     pb = pe;
     pc = pf;
   }
-  if (k < steps) run_step<HasDirty, MaxRing>(A, sg, pa, pb, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
-  if (k + 1 < steps) run_step<HasDirty, MaxRing>(B, sg, pb, pc, barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+  if (k < steps)
+    run_step<HasDirty, MaxRing>(A, sg, pa, pb, pieces.barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
+  if (k + 1 < steps)
+    run_step<HasDirty, MaxRing>(B, sg, pb, pc, pieces.barriers, ring_len, W, ld, dirty_world, rw, rdw, rows, flag);
 }
 
 // dp::math::invertTranspose (dp/math/Matmnt.h:1171-1201) of W[s]: 2x2 minors of
@@ -679,10 +658,11 @@ namespace {
 // Threads of a tile workgroup where the caller leaves them to the plan.  Smaller
 // workgroups split a tree over more CUs, shorten each tile's steps and mix the
 // reads of one tile with the writes of another; larger ones recompute fewer
-// shared ancestors.  Full propagation with 256 / 512 / 1024 threads: 3,000 nodes
-// 6.6 / 6.5 / 7.3 us, 50,000 8.1 / 9.1 / 9.5, 250,007 13.9 / 12.9 / 12.8, 500,000
-// 16.7 / 16.1 / 16.9, 700,000 25.6 / 25.6 / 30.9, 1,000,000 35.4 / 37.4 / 37.3.
-uint32_t default_tile_threads(uint64_t slots) { return slots > 150000 && slots < 600000 ? 512 : 256; }
+// shared ancestors.  Full propagation with 256 / 512 / 1024 threads: 10,000 nodes
+// 5.9 / 5.9 / 6.2 us, 50,000 7.1 / 7.1 / 7.2, 100,000 8.7 / 8.2 / 8.2, 250,007
+// 12.7 / 11.7 / 11.9, 500,000 15.8 / 15.1 / 15.8, 700,000 25.0 / 24.6 / 29.6 (1 %
+// dirty 18.6 / 19.5 / 26.0), 1,000,000 34.4 / 35.8 / 36.1.
+uint32_t default_tile_threads(uint64_t slots) { return slots > 75000 && slots < 600000 ? 512 : 256; }
 constexpr size_t kMaxRunPasses = 32;
 
 template <bool HasDirty>
