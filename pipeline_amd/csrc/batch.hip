@@ -13,11 +13,11 @@
 // objects) result is one lane mask, stored as one 64-bit mask word.  No two items
 // write the same mask word, so no atomics touch the output.
 //
-// What bounds it: with many frusta per object, vector instructions: 60 per
-// frustum and 64 objects with the quick test (55 with two objects per lane), 190
-// when each pair took the exact test.  500,003 objects x 32 frusta: 109 -> 36 us;
-// 64 frusta over 64 groups of 2,097,152 objects: 40 -> 36 us, 4.5 TB/s, now bound
-// by reading the objects.
+// What bounds it: with many frusta per object, vector instructions: 48 per
+// frustum and 64 objects with the quick test (44 with two objects per lane), 190
+// when each pair took the exact test.  500,003 objects x 32 frusta: 109 -> 36 us,
+// of which 25 are the instructions' issue; 64 frusta over 64 groups of 2,097,152
+// objects: 40 -> 36 us, 4.5 TB/s, now bound by reading the objects.
 //
 // Schedule: items are sorted by cost (frusta x objects) on the host, and the
 // persistent grid walks them round-robin (wave w takes w, w+W, ...), which
@@ -161,7 +161,7 @@ __device__ __forceinline__ void quick_objects(const Slot (&slot)[K], const RawOb
 // objects.  Words that the quick test (quick_cull.hpp) decides whole are stored
 // at once, by every lane (the same value to the same address: a store from lane
 // 0 alone would change the exec mask around it); the others wait in the queue.
-// view_of(p, frustum, m) gives the QuickView of the item's p-th frustum; with
+// view_of(p, frustum) gives the QuickView of the item's p-th frustum; with
 // `last` the queue is drained before the return.
 template <int K, class ViewOf>
 __device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObjects<K>& t, uint32_t lane,
@@ -179,7 +179,7 @@ __device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObje
       const KPair q = next;
       Mat16 m;
       load_vp(vps, q.frustum, m);
-      const QuickView view = view_of(p, q.frustum, m);
+      const QuickView& view = view_of(p, q.frustum);
       next = list[p + 1 < item.pair_count ? p + 1 : p];
       unsigned long long bits[K], open[K];
       uint32_t n_open = 0;
@@ -232,12 +232,25 @@ __device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObje
   }
 }
 
-// The QuickViews of a launch's frusta, computed once per workgroup into LDS
-// (Table: at most kTableViews frusta, 6 KB; else each use computes its own).
-// From the matrix in scalar registers a QuickView takes 34 vector and 18 scalar
-// instructions per use, from LDS three broadcast reads.
+// Where a wave finds the QuickViews of its frusta: 38 vector instructions with
+// four square roots and 18 scalar ones would go into each use.  The batched kernel
+// keeps those of all frusta of a launch in LDS, computed once per workgroup (Table:
+// at most kTableViews frusta, 8 KB); without, and in the serving kernel, a wave
+// computes those of the list at hand, one per lane, kWave at a time.
 constexpr uint32_t kTableViews = 128;
 constexpr uint32_t kBatchWaves = 4;  // waves of a workgroup, at most
+
+__device__ __forceinline__ void list_views(const KPair* __restrict__ list, uint32_t count,
+                                           const float* __restrict__ vps, uint32_t lane, QuickView* views)
+{
+  wave_lds_order();
+  if (lane < count) {
+    Mat16 m;
+    load_vp(vps, list[lane].frustum, m);
+    views[lane] = quick_view(m.m);
+  }
+  wave_lds_order();
+}
 
 template <int K, bool Table>
 __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restrict__ items, uint32_t n_items,
@@ -246,7 +259,7 @@ __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restr
                                                          const float* __restrict__ vps, uint32_t n_frusta,
                                                          unsigned long long* __restrict__ masks)
 {
-  __shared__ QuickView table[Table ? kTableViews : 1];
+  __shared__ QuickView table[Table ? kTableViews : kBatchWaves * kWave];
   __shared__ Queue<K> queues[kBatchWaves];
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t waves_per_block = blockDim.x / kWave;
@@ -254,7 +267,6 @@ __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restr
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   uint32_t it = blockIdx.x * waves_per_block + wave;
   uint32_t waiting = 0, words = 0;
-  auto view_of = [&](uint32_t, uint32_t f, const Mat16& m) { return Table ? table[f] : quick_view(m.m); };
   for (bool first = true;; first = false) {
     const WorkItem item = items[it < n_items ? it : 0];  // (n_items >= 1)
     Slot slot[K];
@@ -274,6 +286,11 @@ __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restr
     TileObjects<K> objects;
     quick_objects<K>(slot, raw, objects);
     const bool last = it + n_waves >= n_items;
+    auto view_of = [&](uint32_t p, uint32_t f) -> const QuickView& {
+      if (Table) return table[f];
+      if (p % kWave == 0) list_views(pairs + item.pair_begin + p, item.pair_count - p, vps, lane, &table[wave * kWave]);
+      return table[wave * kWave + p % kWave];
+    };
     test_frusta<K>(item, objects, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, last, view_of);
     if (last) break;
     it += n_waves;
@@ -350,19 +367,13 @@ __global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __res
     RawObj raw[K];
     load_objects<K>(scenes, item, lane, slot, raw);
     if (viewed != a) {  // the entry's QuickViews, one per lane, while its first objects are in flight
-      wave_lds_order();
-      if (lane < e.pair_count) {
-        Mat16 m;
-        load_vp(vps, pairs[e.pair_begin + lane].frustum, m);
-        views[block_wave][lane] = quick_view(m.m);
-      }
-      wave_lds_order();
+      list_views(pairs + e.pair_begin, e.pair_count, vps, lane, views[block_wave]);
       viewed = a;
     }
     TileObjects<K> objects;
     quick_objects<K>(slot, raw, objects);
     test_frusta<K>(item, objects, lane, pairs, scenes, vps, masks, queues[block_wave], waiting, words, !more,
-                   [&](uint32_t p, uint32_t, const Mat16&) { return views[block_wave][p]; });
+                   [&](uint32_t p, uint32_t) -> const QuickView& { return views[block_wave][p]; });
     if (!more) break;
     e = ne;
     a = na;
@@ -483,15 +494,21 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   if (!cfg) {
     // Two objects per lane halve the per-frustum work that a wave does once for all
     // its objects, and halve the waves: worth it where both are plenty (300,000
-    // objects x 32 views: 25.5 us against 26.7 with one; 1,000,000 x 8: 27.3
-    // against 26.1; 150,000 objects, 13,000 (tile, view) pairs: 10.0 against 8.7).
+    // objects x 32 views: 24.0 us against 25.7 with one; 1,000,000 x 8: 26.2
+    // against 25.5; 150,000 objects, 13,000 (tile, view) pairs: 9.9 against 8.8).
+    // The grid is then what the device holds at once, 16 waves per CU: with 24 the
+    // last third starts late (500,003 x 32: 36.4 us against 39.0).
     uint64_t tiles = 0, tile_pairs = 0;
     for (size_t g = 0; g < n_groups; ++g) {
       const uint64_t n = group_pair_begin[g + 1] - group_pair_begin[g], t = (groups[g].count + kWave - 1) / kWave;
       tiles += n ? t : 0;
       tile_pairs += n * t;
     }
-    if (tiles >= 16ull * cus && tile_pairs >= 16 * tiles) plan->cfg.objects_per_lane = c.objects_per_lane = 2;
+    if (tiles >= 16 * cus && tile_pairs >= 16 * tiles) {
+      c.objects_per_lane = 2;
+      c.waves_per_cu = 16;
+      plan->cfg = c;
+    }
   }
   const uint64_t tile_objects = static_cast<uint64_t>(kWave) * c.objects_per_lane;
   if (c.max_frusta_per_item == 0) {

@@ -7,33 +7,42 @@
 // 188 operations.  Its outcome depends on the rounding of those operations only
 // where a corner lies within a rounding error of a plane.  Everywhere else any
 // evaluation with a known error bound gives the same answer: here the clip-space
-// centre of the object's world box (twice the centre, 2p + ex + ey + ez) and the
-// radius of the world-axis-aligned box around it, about 50 operations with
-// fused multiply-adds.  A pair closer to a plane than `eps`, a bound on all
-// rounding errors of both evaluations, is left undecided.
+// centre of the object (twice the centre, 2p + ex + ey + ez) and a sphere around
+// it, 38 operations with fused multiply-adds.  A pair closer to a plane than
+// `eps`, a bound on all rounding errors of both evaluations, is left undecided, and
+// so is one whose sphere reaches a plane that its centre lies outside of: 2 to 10
+// in a thousand of the pairs of ordinary scenes, most of which do touch a plane.
 //
 // In terms of the exact sums over the eight corners, with w and c (= x, y or z)
 // the clip coordinates, the reference reports an object culled when on some axis
 // all corners have c <= -w, or all have w <= c and none has c <= -w.
 //   visible   the centre lies inside all six planes: some corner then lies
 //             strictly inside each of them
-//   culled    x, y: |c| - radius(c) > |w| + radius(w): every corner is beyond the
-//             same plane, and (for c > 0) no corner has c <= -w
+//   culled    x, y: |c| - |w| > r max(|Mw - Mc|, |Mw + Mc|) at the centre: every
+//             corner is beyond the same plane, and (for c > 0) none has c <= -w
 //             z: every corner has z < -w; or every corner has w < z and z > -w
+// (Mc: the first three elements of a column of the matrix; r: the sphere's radius.)
 // z uses the sums z + w and w - z of the matrix's columns: for a distant far
 // plane w - z hardly changes with the position, while z and w do.
+//
+// The sphere (doubled scale): |+-ex +-ey +-ez|^2 is at most the sum of the edges'
+// squares and twice the magnitudes of their products, which for the edges of a box
+// under rotation and scale are zero.  Radius and norms are rounded up: by 2^-18 of
+// their value, over ten times what their evaluation can lose, and by 2^-60, more
+// than the underflow of squares hides.
 //
 // The bound.  u = 2^-24, A_j = |p_j| + |ex_j| + |ey_j| + |ez_j|, S_c = sum_j A_j
 // |M_jc|, everything in the doubled scale.  Errors of the exact test's corners:
 // 14 u S_c per coordinate (four-term products 4 u, three adds 3 u, doubled).
-// Errors here: centre 12 u S_c, radii and chained sums 11 u S_c, the column sums
-// and last adds 4 u more: below 41 u (S_c + S_w) together.  S_c + S_w <=
-// 2 (n3 * s3 + n4 * sw) with n3, n4 the largest magnitudes of rows 0-2 and row 3
-// and s3 = sum of A_j over x, y, z, sw = A_w.  eps = 2^-17 (n3 s3 + n4 sw) = 64 u
-// (S_c + S_w)'s bound.  The added 2^-117 and 2^-130 cover underflow.  Operands
-// of 2^56 (matrix) or 2^60 (object) and above, infinities and NaN make eps
-// infinite or NaN, and every comparison below false: undecided.  So does an
-// object whose edges have a w component.
+// Errors here: centre 12 u S_c per coordinate, or 14 u (S_z + S_w) by the column
+// sums, and 4 u (S_c + S_w) of the last adds: 30 u (S_c + S_w) together.  S_c + S_w
+// <= 2 (n3 * s3 + n4 * sw) with n3, n4 the largest magnitudes of rows 0-2 and row 3,
+// s3 >= sum of A_j over x, y, z (the edges' part is at most 3 r), sw = A_w; the
+// differences of columns inside the norms lose at most 12 u n3 s3 more.  eps = 2^-17
+// (n3 s3 + n4 sw) = 128 u (n3 s3 + n4 sw) against those 72.  The added 2^-117 and
+// 2^-130 cover underflow.  Operands of 2^56 (matrix) or 2^60 (object) and above,
+// infinities and NaN make eps infinite or NaN, and every comparison below false:
+// undecided.  So does an object whose edges have a w component.
 #pragma once
 
 #include <cstdint>
@@ -49,18 +58,35 @@ namespace dpc {
 // What the quick test reads of an object (doubled scale).
 struct QuickObj {
   float cx, cy, cz, cw;  // 2p + ex + ey + ez
-  float hx, hy, hz;      // |ex| + |ey| + |ez| per component
+  float r;               // radius of a sphere around it that holds the object
   float s3, sw;          // the object's factors of eps
 };
 
 // What it reads of a view-projection matrix beside its elements.
 struct alignas(16) QuickView {
-  float lo[4], hi[4];  // rows of z + w and w - z
-  float n3, n4;        // largest magnitude in rows 0-2, in row 3 (infinite from 2^56 on)
+  float lo[4], hi[4];    // rows of z + w and w - z
+  float nx, ny, nl, nh;  // norms: of w - x or w + x, of w - y or w + y (the larger), of z + w, of w - z
+  float n3, n4;          // largest magnitude in rows 0-2, in row 3 (infinite from 2^56 on)
   float pad[2];
 };
 
 DPC_HD float quick_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// A square root of v or more (v >= 0, or NaN).
+DPC_HD float quick_root(float v)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+  const float root = __builtin_amdgcn_sqrtf(v);  // (within an ulp, like the correctly rounded one)
+#else
+  const float root = __builtin_sqrtf(v);
+#endif
+  return quick_fma(root, 1.0f + 0x1p-18f, 0x1p-60f);
+}
+
+DPC_HD float quick_dot(float ax, float ay, float az, float bx, float by, float bz)
+{
+  return quick_fma(az, bz, quick_fma(ay, by, ax * bx));
+}
 
 // p, ex, ey, ez: the object's point and edges as the exact test takes them.
 template <class V4>
@@ -71,12 +97,15 @@ DPC_HD QuickObj quick_obj(const V4& p, const V4& ex, const V4& ey, const V4& ez)
   q.cy = quick_fma(2.0f, p.y, (ex.y + ey.y) + ez.y);
   q.cz = quick_fma(2.0f, p.z, (ex.z + ey.z) + ez.z);
   q.cw = 2.0f * p.w;
-  q.hx = (__builtin_fabsf(ex.x) + __builtin_fabsf(ey.x)) + __builtin_fabsf(ez.x);
-  q.hy = (__builtin_fabsf(ex.y) + __builtin_fabsf(ey.y)) + __builtin_fabsf(ez.y);
-  q.hz = (__builtin_fabsf(ex.z) + __builtin_fabsf(ey.z)) + __builtin_fabsf(ez.z);
+  const float squares = (quick_dot(ex.x, ex.y, ex.z, ex.x, ex.y, ex.z) + quick_dot(ey.x, ey.y, ey.z, ey.x, ey.y, ey.z)) +
+                        quick_dot(ez.x, ez.y, ez.z, ez.x, ez.y, ez.z);
+  const float products = (__builtin_fabsf(quick_dot(ex.x, ex.y, ex.z, ey.x, ey.y, ey.z)) +
+                          __builtin_fabsf(quick_dot(ey.x, ey.y, ey.z, ez.x, ez.y, ez.z))) +
+                         __builtin_fabsf(quick_dot(ez.x, ez.y, ez.z, ex.x, ex.y, ex.z));
+  q.r = quick_root(quick_fma(2.0f, products, squares));
   const float flat = (__builtin_fabsf(ex.w) + __builtin_fabsf(ey.w)) + __builtin_fabsf(ez.w);
   const float aw = __builtin_fabsf(p.w);
-  const float a3 = ((__builtin_fabsf(p.x) + __builtin_fabsf(p.y)) + __builtin_fabsf(p.z)) + ((q.hx + q.hy) + q.hz);
+  const float a3 = quick_fma(3.0f, q.r, (__builtin_fabsf(p.x) + __builtin_fabsf(p.y)) + __builtin_fabsf(p.z));
   const bool fits = (flat == 0.0f) & (a3 + aw < 0x1p60f);  // (false for NaN)
   q.s3 = fits ? quick_fma(a3, 0x1p-17f, 0x1p-117f) : __builtin_inff();
   q.sw = quick_fma(aw, 0x1p-17f, 0x1p-117f);
@@ -101,6 +130,17 @@ DPC_HD QuickView quick_view(const float* m)
     v.lo[j] = m[4 * j + 2] + m[4 * j + 3];
     v.hi[j] = m[4 * j + 3] - m[4 * j + 2];
   }
+  v.nl = quick_root(quick_dot(v.lo[0], v.lo[1], v.lo[2], v.lo[0], v.lo[1], v.lo[2]));
+  v.nh = quick_root(quick_dot(v.hi[0], v.hi[1], v.hi[2], v.hi[0], v.hi[1], v.hi[2]));
+  float n[2];
+  for (int c = 0; c < 2; ++c) {
+    const float d0 = m[3] - m[c], d1 = m[7] - m[4 + c], d2 = m[11] - m[8 + c];
+    const float s0 = m[3] + m[c], s1 = m[7] + m[4 + c], s2 = m[11] + m[8 + c];
+    const float d = quick_dot(d0, d1, d2, d0, d1, d2), s = quick_dot(s0, s1, s2, s0, s1, s2);
+    n[c] = quick_root(d > s ? d : s);  // (NaN: n3 is NaN too)
+  }
+  v.nx = n[0];
+  v.ny = n[1];
   uint32_t n3 = 0, n4 = 0;
   for (int k = 0; k < 12; ++k) {
     const uint32_t b = quick_magnitude(m[k]);
@@ -137,22 +177,11 @@ DPC_HD QuickResult<M> quick_test(const QuickObj& q, const float* m, const QuickV
   const float dl = quick_fma(q.cw, v.lo[3], quick_fma(q.cz, v.lo[2], quick_fma(q.cy, v.lo[1], q.cx * v.lo[0])));
   const float dh = quick_fma(q.cw, v.hi[3], quick_fma(q.cz, v.hi[2], quick_fma(q.cy, v.hi[1], q.cx * v.hi[0])));
   const float acx = __builtin_fabsf(cx), acy = __builtin_fabsf(cy);
-  // radius(x) - |x|, radius(y) - |y|, |w| + radius(w), radius(z + w), (w - z) + radius(w - z)
-  const float rx = quick_fma(q.hz, __builtin_fabsf(m[8]),
-                             quick_fma(q.hy, __builtin_fabsf(m[4]), quick_fma(q.hx, __builtin_fabsf(m[0]), -acx)));
-  const float ry = quick_fma(q.hz, __builtin_fabsf(m[9]),
-                             quick_fma(q.hy, __builtin_fabsf(m[5]), quick_fma(q.hx, __builtin_fabsf(m[1]), -acy)));
-  const float rw = quick_fma(q.hz, __builtin_fabsf(m[11]),
-                             quick_fma(q.hy, __builtin_fabsf(m[7]),
-                                       quick_fma(q.hx, __builtin_fabsf(m[3]), __builtin_fabsf(cw))));
-  const float rl = quick_fma(q.hz, __builtin_fabsf(v.lo[2]),
-                             quick_fma(q.hy, __builtin_fabsf(v.lo[1]), q.hx * __builtin_fabsf(v.lo[0])));
-  const float rh = quick_fma(q.hz, __builtin_fabsf(v.hi[2]),
-                             quick_fma(q.hy, __builtin_fabsf(v.hi[1]), quick_fma(q.hx, __builtin_fabsf(v.hi[0]), dh)));
-  const float inner = cw - eps, outer = rw + eps;
+  const float inner = cw - eps, outer = __builtin_fabsf(cw) + eps;
   QuickResult<M> r;
   r.visible = less(acx, inner) & less(acy, inner) & less(eps, dl) & less(eps, dh);
-  r.culled = less(outer, -rx) | less(outer, -ry) | less(dl + rl, -eps) | (less(rh, -eps) & less(eps, dl - rl));
+  r.culled = less(quick_fma(q.r, v.nx, outer), acx) | less(quick_fma(q.r, v.ny, outer), acy) |
+             less(quick_fma(q.r, v.nl, dl), -eps) | (less(quick_fma(q.r, v.nh, dh), -eps) & less(eps, quick_fma(-q.r, v.nl, dl)));
   return r;
 }
 
