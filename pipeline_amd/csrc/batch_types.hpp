@@ -42,13 +42,25 @@ constexpr uint32_t kMaxHostScatterLd = (1u << 26) - 1;
 int launch_scatter_host(float* d_planes, size_t ld, const uint32_t* idx, const float* src, size_t count,
                         void* stream);
 
-// Scatters count delta matrices that crossed PCIe packed (device memory, 16-byte
-// aligned): matrix k as three 16-byte rows in d_packed, (row i's x y z, row 3's
-// component i) for i = 0, 1, 2, and its last column (m[3], m[7], m[11], m[15])
-// as 16 bytes in d_tails, or, with d_tails null, 0 0 0 1 for every matrix.
-// Every value is moved as its bits.
-int launch_scatter_affine(float* d_planes, size_t ld, const uint32_t* d_idx, const void* d_packed,
-                          const void* d_tails, size_t count, void* stream);
+// One packed delta of a batch's arena (byte offsets, 16-byte aligned): count
+// indices; matrix k as three 16-byte rows, (row i's x y z, row 3's component i)
+// for i = 0, 1, 2; and the last columns (m[3], m[7], m[11], m[15]) as 16 bytes
+// each, or, with tails 0, 0 0 0 1 for every matrix.  Its matrices go to `planes`
+// (row planes of ld slots); every value is moved as its bits.
+struct StageJob {
+  float* planes;
+  uint64_t ld;
+  uint32_t idx, packed, tails;
+  uint32_t count;
+};
+static_assert(sizeof(StageJob) == 32, "StageJob layout");
+
+// Scatters the n jobs' deltas out of an arena of `bytes` bytes (below 2^31).  With
+// d_arena set the arena lies in pinned host memory and its first desc_bytes bytes
+// (a multiple of 16) are copied to d_arena as well: a batch's whole upload in one
+// launch.  With d_arena null it is device memory, and the deltas are scattered only.
+int launch_stage(const char* arena, uint64_t bytes, char* d_arena, uint64_t desc_bytes, const StageJob* jobs, uint32_t n,
+                 void* stream);
 
 // One request's masks to its caller's buffer in pinned host memory: `words`
 // 64-bit words from byte offset src_offset of the batch arena to dst (the

@@ -57,6 +57,14 @@ constexpr uint64_t kHostArena = 4096 + kMaxBatch * 32 + kMaxBatch * kMaxFrusta *
 constexpr uint64_t kHostStageMax = 32ull << 20;
 // a delta's matrices up to this size are staged; a larger array is copied on its own
 constexpr uint64_t kStageMatsMax = kHostStageMax;
+// A batch that stages up to this many bytes is uploaded by the kernel that scatters
+// its deltas (dpc::launch_stage), a larger one by a DMA copy before it: beside the
+// masks on their way out a kernel reads host memory at half the copy's rate, but it
+// waits for no signal.  One request for each of 16 scenes, 1 KB to 2 MB staged: 382
+// to 396 us with the line at 256 KiB to 8 MiB, 417 to 424 with copies only; 20,000
+// requests/s offered, mean 1.7 MB: 186 to 189 G tests/s with copies only and with a
+// line at 1 MiB, 181 at 3, 159 at 8.
+constexpr uint64_t kStageRead = 1ull << 20;
 
 uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
 
@@ -271,6 +279,7 @@ struct StreamSlot {
   hipEvent_t done = nullptr;
   char* d_arena = nullptr;
   char* h_arena = nullptr;  // pinned, h_cap bytes: the device arena's first h_cap bytes staged on the host
+  const char* h_arena_dev = nullptr;  // its device-visible address
   uint64_t cap = 0;
   uint64_t h_cap = 0;
   bool busy = false;     // formed and not yet completed
@@ -521,8 +530,9 @@ void dpc_server::issue_batch(StreamSlot& slot)
   double copy_us = 0.0;
   t_part[0] = now();
   // The descriptors, the index arrays and the smaller matrix arrays (packed)
-  // staged together in the pinned host arena when they fit: one copy for them,
-  // then the larger matrix arrays on their own, then the scatters.  Otherwise
+  // staged together in the pinned host arena when they fit: one launch that
+  // uploads and scatters them, or one copy and a scatter launch, then the larger
+  // matrix arrays on their own.  Otherwise
   // each delta is copied on its own, before its scatter.
   std::vector<std::atomic<bool>> nonaffine(pick.size());  // (all false)
   if (staged) {
@@ -536,15 +546,34 @@ void dpc_server::issue_batch(StreamSlot& slot)
                                slot.h_arena + tail_off[k], &nonaffine[k]});
     }
     gather(pool, pieces);
-    bool tails = false;
-    for (auto& f : nonaffine) tails = tails || f.load(std::memory_order_relaxed);
-    if (rc == DPC_OK) {
-      e = hipMemcpyAsync(slot.d_arena, slot.h_arena, tails ? stage_end : packed_end, hipMemcpyHostToDevice, s);
+    bool tails = false, whole = true;  // whole: no delta of the batch is copied on its own
+    std::vector<dpc::StageJob> jobs;
+    for (size_t k = 0; k < pick.size(); ++k) {
+      const Request& r = *pick[k];
+      if (!r.n_delta || r.didx_dev) continue;
+      if (64ull * r.n_delta > kStageMatsMax) {
+        whole = false;
+        continue;
+      }
+      const bool tail = nonaffine[k].load(std::memory_order_relaxed);
+      tails = tails || tail;
+      jobs.push_back(dpc::StageJob{snapshot[k].planes, snapshot[k].n_mat, static_cast<uint32_t>(idx_off[k]),
+                                   static_cast<uint32_t>(mat_off[k]), tail ? static_cast<uint32_t>(tail_off[k]) : 0u,
+                                   r.n_delta});
+      if (!tail) pick[k]->delta_packed = true;
+    }
+    const uint64_t bytes = tails ? stage_end : packed_end;
+    const bool read = whole && bytes <= kStageRead && slot.h_arena_dev;
+    if (rc == DPC_OK && !read) {
+      e = hipMemcpyAsync(slot.d_arena, slot.h_arena, bytes, hipMemcpyHostToDevice, s);
       if (e != hipSuccess) rc = hip_fail(e, "batch upload");
     }
     copy_us = now() - t_part[0];
+    if (rc == DPC_OK)
+      rc = dpc::launch_stage(read ? slot.h_arena_dev : slot.d_arena, bytes, read ? slot.d_arena : nullptr,
+                             read ? desc_end : 0, jobs.data(), static_cast<uint32_t>(jobs.size()), s);
   }
-  // deltas: copy to the device (unless staged above) and scatter into the scenes' matrices
+  // the other deltas: copy to the device and scatter into the scenes' matrices
   for (size_t k = 0; k < pick.size() && rc == DPC_OK; ++k) {
     const Request& r = *pick[k];
     if (!r.n_delta) continue;
@@ -552,15 +581,7 @@ void dpc_server::issue_batch(StreamSlot& slot)
       rc = dpc::launch_scatter_host(snapshot[k].planes, snapshot[k].n_mat, r.didx_dev, r.dmats_dev, r.n_delta, s);
       continue;
     }
-    if (staged && 64ull * r.n_delta <= kStageMatsMax) {
-      const bool tail = nonaffine[k].load(std::memory_order_relaxed);
-      rc = dpc::launch_scatter_affine(snapshot[k].planes, snapshot[k].n_mat,
-                                      reinterpret_cast<const uint32_t*>(slot.d_arena + idx_off[k]),
-                                      slot.d_arena + mat_off[k], tail ? slot.d_arena + tail_off[k] : nullptr,
-                                      r.n_delta, s);
-      if (!tail) pick[k]->delta_packed = true;
-      continue;
-    }
+    if (staged && 64ull * r.n_delta <= kStageMatsMax) continue;  // (scattered above)
     {
       const double tc = now();
       if (!staged) e = hipMemcpyAsync(slot.d_arena + idx_off[k], r.didx, 4ull * r.n_delta, hipMemcpyHostToDevice, s);
@@ -766,6 +787,7 @@ int dpc_server_create(const dpc_server_config* cfg, dpc_server** out)
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&sl.d_arena), per);
     sl.h_cap = std::max(kHostArena, std::min(per, kHostStageMax));
     if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&sl.h_arena), sl.h_cap, hipHostMallocDefault);
+    if (e == hipSuccess) sl.h_arena_dev = static_cast<const char*>(pinned_range(sl.h_arena, sl.h_cap));
     sl.cap = per;
   }
   if (e != hipSuccess) {

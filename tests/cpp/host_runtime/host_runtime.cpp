@@ -179,6 +179,14 @@ int launch_scatter_affine(float* planes, size_t ld, const uint32_t* idx, const v
   }
   return DPC_OK;
 }
+int launch_stage(const char* arena, uint64_t, char* d_arena, uint64_t desc_bytes, const StageJob* jobs, uint32_t n, void*)
+{
+  if (d_arena) std::memcpy(d_arena, arena, desc_bytes);
+  for (uint32_t k = 0; k < n; ++k)
+    launch_scatter_affine(jobs[k].planes, jobs[k].ld, reinterpret_cast<const uint32_t*>(arena + jobs[k].idx),
+                          arena + jobs[k].packed, jobs[k].tails ? arena + jobs[k].tails : nullptr, jobs[k].count, nullptr);
+  return DPC_OK;
+}
 int launch_copy_out(const void*, uint32_t, const char*, uint64_t, void*) { return DPC_OK; }
 }  // namespace dpc
 
