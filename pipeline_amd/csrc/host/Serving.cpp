@@ -689,26 +689,34 @@ void dpc_server::run()
 {
   (void)hipSetDevice(device);
   std::unique_lock<std::mutex> lock(mu);
+  std::vector<std::pair<size_t, hipError_t>> watched;  // issued slots and their events' states
   for (;;) {
     bool progressed = false;
     bool any_busy = false;
-    for (auto& slot : slots) {
-      if (slot.busy && !slot.issued) {
-        any_busy = true;  // its issuer is making the calls
-      } else if (slot.busy) {
-        const hipError_t q = hipEventQuery(slot.done);
-        if (q == hipSuccess) {
+    watched.clear();
+    for (size_t k = 0; k < slots.size(); ++k) {
+      if (!slots[k].busy) continue;
+      any_busy = true;
+      if (slots[k].issued) watched.push_back({k, hipErrorNotReady});  // (otherwise its issuer is making the calls)
+    }
+    if (!watched.empty()) {
+      // The events are queried without the lock, a microsecond or more each:
+      // callers that submit would wait for it.  (An issued slot changes only here.)
+      lock.unlock();
+      for (auto& w : watched) w.second = hipEventQuery(slots[w.first].done);
+      lock.lock();
+      for (const auto& w : watched) {
+        StreamSlot& slot = slots[w.first];
+        if (w.second == hipSuccess) {
           complete(slot);
           progressed = true;
-        } else if (q != hipErrorNotReady) {
+        } else if (w.second != hipErrorNotReady) {
           // the batch cannot be observed to finish (the device reported an
           // error): its requests fail instead of waiting for ever
           (void)hipGetLastError();
           for (auto& r : slot.reqs) r->status = DPC_ERR_HIP;
           complete(slot);
           progressed = true;
-        } else {
-          any_busy = true;
         }
       }
     }
@@ -962,6 +970,9 @@ int dpc_server_submit(dpc_server* s, uint32_t scene_id, const float* vps, uint32
       r->dmats_dev = static_cast<const float*>(dm);
     }
   }
+  // the largest delta index, found before the lock is taken
+  uint32_t top = 0;
+  for (uint32_t k = 0; k < n_delta; ++k) top = std::max(top, didx[k]);
   std::lock_guard<std::mutex> g(s->mu);
   // (a scene still being uploaded has no id for its caller yet, and no sizes)
   if (scene_id >= s->scenes.size() || !s->scenes[scene_id].live || !s->scenes[scene_id].ready)
@@ -972,8 +983,7 @@ int dpc_server_submit(dpc_server* s, uint32_t scene_id, const float* vps, uint32
     r->dmats_dev = nullptr;
   }
   // delta indices are checked here, on the host, so the scatter never writes outside the scene
-  for (uint32_t k = 0; k < n_delta; ++k)
-    if (didx[k] >= sc.n_mat) return fail(DPC_ERR_INVALID_ARGUMENT, "dpc_server_submit: delta index out of range");
+  if (n_delta && top >= sc.n_mat) return fail(DPC_ERR_INVALID_ARGUMENT, "dpc_server_submit: delta index out of range");
   r->words = (sc.n + 63) / 64;
   if (mask_capacity_words < r->words * n_frusta)
     return fail(DPC_ERR_INVALID_ARGUMENT, "dpc_server_submit: the mask buffer is smaller than n_frusta x ceil(n/64) words");

@@ -201,9 +201,14 @@ def upload_scene(lower: np.ndarray, upper: np.ndarray, matrices: np.ndarray,
     return DeviceScene(box_a, box_b, planes, ld, n, dx)
 
 
+_Mat16 = C.c_float * 16
+
+
 def vp_arg(vp: np.ndarray):
-    v = np.ascontiguousarray(vp, np.float32).reshape(16)
-    return (C.c_float * 16)(*v.tolist())
+    v = np.ascontiguousarray(vp, np.float32)
+    if v.size != 16:
+        raise ValueError(f"a view-projection matrix has 16 elements, not {v.size}")
+    return _Mat16.from_buffer_copy(v)  # (one copy: sixteen Python floats took 1.5 us more, a fifth of a small cull)
 
 
 def cull(scene: DeviceScene, vp: np.ndarray, out: DeviceArray | None = None, stream=None) -> DeviceArray:
