@@ -8,6 +8,7 @@
 #include <atomic>
 #include <cfloat>
 #include <mutex>
+#include <type_traits>
 
 #include "cull_math.hpp"
 #include "internal.hpp"
@@ -446,9 +447,18 @@ __device__ __forceinline__ BoxIn load_box_in(const float4* __restrict__ box_a, c
 // What bounds it: reading the objects.  Beside that, minima and maxima of values
 // take 36 instructions per object and 80 per wave, where an extremum with its
 // object's index took 120 and, through LDS permutes, 430.  A call over 2,400,000
-// objects in the order of their matrices: 29.4 -> 25.8 us (104 MB; the cull that
-// reads the same takes 24.0); 600,011: 13.9 -> 11.3; the same with matrices at
-// random 41.6 -> 40.0, where each object's four rows are 128-byte lines of their own.
+// objects in the order of their matrices: 29.4 -> 25.9 us (104 MB; the cull that
+// reads the same takes 24.0); 600,011: 13.9 -> 11.3.
+//
+// With matrices in no order each row is a 128-byte line of its own, shared only
+// with other objects' rows of the same plane.  A wave that finds its first 64
+// matrices in 32 lines or more therefore takes up to three rounds at once, row by
+// row: all waves read one plane at a time, and of a plane, unlike of four, an XCD's
+// L2 holds a good part (600,011 objects over 200,003 matrices, 3.2 MB a plane: 46 %
+// of the reads hit instead of 28 %, 40.0 -> 33.2 us; 400,000: 25.7 -> 20.4; 250,000,
+// a round per wave: 14.7 -> 13.8; 2,400,000: 171 -> 163).  In order, where the reads
+// share their lines, that waits more often (2,400,000 objects: 29.4 us against 25.9;
+// 250,000: 10.1 against 8.4), so those waves keep two sets of inputs in turn.
 template <bool Indexed>
 __global__ __launch_bounds__(kBoxThreads) void bbox_partial_kernel(const float4* __restrict__ box_a,
                                                                    const float2* __restrict__ box_b,
@@ -479,10 +489,8 @@ __global__ __launch_bounds__(kBoxThreads) void bbox_partial_kernel(const float4*
   // Folds an object (index i, matrix m, inputs d) into the lane's box.  A lane past
   // the chunk's end has the chunk's first object, which changes nothing; an object
   // whose matrix index is outside the array adds nothing.
-  auto fold = [&](const BoxIn& d, size_t i, size_t m) {
-    if (m >= ld) return;
+  auto fold_obb = [&](const Obb& o, size_t i) {
     // ManagerBitSet.cpp:282-294: v0 = lower * M, x/y/z = extent[k] * row k, same add tree as the cull.
-    const Obb o = make_obb(d.a, d.b, d.r0, d.r1, d.r2, d.r3);
     float4 v[8];
     v[0] = o.p;
     v[1] = add4(o.p, o.ex);
@@ -512,7 +520,67 @@ __global__ __launch_bounds__(kBoxThreads) void bbox_partial_kernel(const float4*
       }
     }
   };
-  if (rounds) {
+  auto fold = [&](const BoxIn& d, size_t i, size_t m) {
+    if (m < ld) fold_obb(make_obb(d.a, d.b, d.r0, d.r1, d.r2, d.r3), i);
+  };
+  size_t done = 0;  // rounds
+  // K rounds of scattered matrices, row by row
+  auto fold_rows = [&](auto rounds_at_once) {
+    constexpr int K = decltype(rounds_at_once)::value;
+    size_t m[K];
+    float4 ba[K], row[K];
+    float2 bb[K];
+    Obb o[K];
+    for (int k = 0; k < K; ++k) {
+      const size_t i = object_of(done + k);
+      m[k] = matrix_of(i);
+      ba[k] = box_a[i];
+      bb[k] = box_b[i];
+    }
+    auto load_row = [&](int r) {
+      for (int k = 0; k < K; ++k) row[k] = planes[r * ld + (m[k] < ld ? m[k] : 0)];
+    };
+    // (the next row's address waits for this row's arithmetic: the compiler would
+    // issue all the loads at once)
+    auto wait_row = [&] {
+      for (int k = 0; k < K; ++k) asm volatile("" : "+v"(m[k]) : "v"(o[k].p.x));
+    };
+    // make_obb row by row: the same products and sums in the same order
+    load_row(0);
+    for (int k = 0; k < K; ++k) {
+      o[k].p = scale4(ba[k].x, row[k]);
+      o[k].ex = scale4(ba[k].w, row[k]);
+    }
+    wait_row();
+    load_row(1);
+    for (int k = 0; k < K; ++k) {
+      o[k].p = add4(o[k].p, scale4(ba[k].y, row[k]));
+      o[k].ey = scale4(bb[k].x, row[k]);
+    }
+    wait_row();
+    load_row(2);
+    for (int k = 0; k < K; ++k) {
+      o[k].p = add4(o[k].p, scale4(ba[k].z, row[k]));
+      o[k].ez = scale4(bb[k].y, row[k]);
+    }
+    wait_row();
+    load_row(3);
+    for (int k = 0; k < K; ++k) {
+      o[k].p = add4(o[k].p, row[k]);
+      if (m[k] < ld) fold_obb(o[k], object_of(done + k));
+    }
+    done += K;
+  };
+  bool scattered = false;
+  if (Indexed && rounds) {
+    const uint32_t line = static_cast<uint32_t>(matrix_of(object_of(0)) / 8);
+    scattered = __popcll(ballot(line != dpp_from<0x138, 0xf>(line))) >= kWave / 2;  // (wave_shr:1)
+  }
+  if (scattered) {
+    while (done + 3 <= rounds) fold_rows(std::integral_constant<int, 3>{});
+    if (done + 2 == rounds) fold_rows(std::integral_constant<int, 2>{});
+    if (done + 1 == rounds) fold_rows(std::integral_constant<int, 1>{});
+  } else if (rounds) {
     size_t ia = object_of(0), ma = matrix_of(ia);
     BoxIn a = load_box_in(box_a, box_b, planes, ld, ia, ma);
     size_t in = object_of(1), mn = matrix_of(in);  // the next round's object and matrix index
