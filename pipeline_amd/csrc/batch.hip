@@ -7,23 +7,25 @@
 // Work decomposition: a group is split into tiles of 64*K objects.  A work item
 // is (tile, slice of the frusta paired with the tile's group).  A wave owns one
 // item at a time: every lane builds what the quick test needs of its K objects
-// once (one read of each object's matrix and box), then the wave loops over the
-// item's frusta.  Each frustum's matrix is wave-uniform, so it is read through
-// the scalar cache into SGPRs and feeds the VALU directly; each (frustum, 64
-// objects) result is one lane mask, stored as one 64-bit mask word.  No two items
-// write the same mask word, so no atomics touch the output.
+// once (one read of each object's matrix and box), then the wave takes the item's
+// frusta in runs of sixteen: the lanes hold four rows of each of the run's views,
+// the matrix cores contract them with the lanes' objects, and each (frustum, 64
+// objects) result is one lane mask, a 64-bit mask word.  No two items write the
+// same mask word, so no atomics touch the output.
 //
-// What bounds it: with many frusta per object, vector instructions: 48 per
-// frustum and 64 objects with the quick test (44 with two objects per lane), 190
-// when each pair took the exact test.  500,003 objects x 32 frusta: 109 -> 36 us,
-// of which 25 are the instructions' issue; 64 frusta over 64 groups of 2,097,152
-// objects: 40 -> 36 us, 4.5 TB/s, now bound by reading the objects.
+// What bounds it: with many frusta per object, instruction issue and what does not
+// overlap it: a frustum and 64 objects take 7 matrix and 13 vector instructions (48
+// vector instructions with the quick test's products on the vector unit, 190 when
+// each pair took the exact test).  500,003 objects x 32 frusta: 109 us with the
+// exact test, 35 with the quick test, 26 with its products on the matrix cores, of
+// which 9 are reading the objects and 10 the instructions; 64 frusta over 64 groups
+// of 2,097,152 objects: 40 -> 36 us, 4.5 TB/s, bound by reading the objects.
 //
 // Schedule: items are sorted by cost (frusta x objects) on the host, and the
 // persistent grid walks them round-robin (wave w takes w, w+W, ...), which
 // bounds the load imbalance by the cost of one item.  Objects are not loaded
-// ahead of the item that is tested: without the 22 registers that takes, seven
-// waves run per SIMD instead of five, and hide the loads themselves.
+// ahead of the item that is tested: without the 22 registers that takes, six
+// waves run per SIMD, and hide the loads themselves.
 #include <algorithm>
 #include <cstring>
 #include <numeric>
@@ -157,86 +159,147 @@ __device__ __forceinline__ void quick_objects(const Slot (&slot)[K], const RawOb
   }
 }
 
-// Tests a work item against its frusta, one mask word per frustum and 64
-// objects.  Words that the quick test (quick_cull.hpp) decides whole are stored
-// at once, by every lane (the same value to the same address: a store from lane
-// 0 alone would change the exec mask around it); the others wait in the queue.
-// view_of(p, frustum) gives the QuickView of the item's p-th frustum; with
+// The entries of a work item's list that a wave's lanes hold: lane 4 f + i that of
+// frustum p0 + f (the last one again past the end).
+__device__ __forceinline__ KPair load_pairs(const KPair* __restrict__ pairs, const WorkItem& item, uint32_t p0,
+                                            uint32_t lane)
+{
+  const uint32_t p = p0 + lane / 4 % kQuickRun;
+  return pairs[item.pair_begin + (p < item.pair_count ? p : item.pair_count - 1)];
+}
+
+template <int Lane>
+__device__ __forceinline__ uint32_t lane_of(uint32_t v)
+{
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), Lane));
+}
+
+// `to` with the wave-uniform v in one lane.
+template <int Lane>
+__device__ __forceinline__ uint32_t set_lane(uint32_t v, uint32_t to)
+{
+  asm("v_writelane_b32 %0, %1, %2" : "+v"(to) : "s"(v), "n"(Lane));
+  return to;
+}
+
+// A run of kQuickRun frusta (at most) of a work item's list.
+template <int K>
+struct Run {
+  uint32_t todo, again;   // bit f: frustum f is to be tested; is to be tested once the queue is empty
+  uint32_t queued[K];     // bit f: word k of frustum f waits in the queue
+  uint32_t lo[K], hi[K];  // lane 4 f: word k of frustum f
+};
+
+// Tests the wave's objects against frustum F of a run.  A word with undecided
+// objects goes to the queue; without room for them the frustum and those after it
+// are left for `again`.
+template <int F, int K>
+__device__ __forceinline__ void test_frustum(Run<K>& run, const WorkItem& item, const TileObjects<K>& t,
+                                             const QuickRows& rows, const KPair& pair, uint32_t lane, Queue<K>& queue,
+                                             uint32_t& waiting, uint32_t& words)
+{
+  if (!((run.todo >> F) & 1)) return;
+  unsigned long long bits[K], open[K], any = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const QuickResult<unsigned long long> r = quick_wave<F>(t.quick[k], rows);
+    bits[k] = (r.visible & t.tested[k]) | t.always[k];
+    open[k] = t.tested[k] & ~(r.visible | r.culled);
+    any |= open[k];
+    run.lo[k] = set_lane<4 * F>(static_cast<uint32_t>(bits[k]), run.lo[k]);
+    run.hi[k] = set_lane<4 * F>(static_cast<uint32_t>(bits[k] >> 32), run.hi[k]);
+  }
+  if (__builtin_expect(any == 0, 1)) return;
+  uint32_t n_open = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) n_open += static_cast<uint32_t>(__builtin_popcountll(open[k]));
+  if (waiting + n_open > Queue<K>::kCapacity) {
+    run.again = run.todo & (~0u << F);
+    run.todo = 0;
+    return;
+  }
+  const uint32_t frustum = lane_of<4 * F>(pair.frustum);
+  const uint64_t word = static_cast<uint64_t>(lane_of<4 * F>(static_cast<uint32_t>(pair.mask_word >> 32))) << 32 |
+                        lane_of<4 * F>(static_cast<uint32_t>(pair.mask_word));
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    if (open[k] == 0) continue;
+    if ((open[k] >> lane) & 1) {
+      const uint64_t object = item.first_object + lane + kWave * k;
+      const uint32_t at = waiting + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(open[k] >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(open[k]), 0u));
+      queue.entry[at] = QueueEntry{static_cast<uint32_t>(object),
+                                   static_cast<uint32_t>(object >> 32) | (words << 16) | (lane << 24), frustum, item.scene};
+    }
+    queue.word[words] = QueueWord{bits[k], word + item.tile_word + k};  // (every lane the same)
+    run.queued[k] |= 1u << F;
+    waiting += static_cast<uint32_t>(__builtin_popcountll(open[k]));
+    ++words;
+  }
+}
+
+// (A matrix instruction names the view it reads, so each frustum of a run has code
+// of its own.)
+template <int F, int K>
+__device__ __forceinline__ void test_run(Run<K>& run, const WorkItem& item, const TileObjects<K>& t,
+                                         const QuickRows& rows, const KPair& pair, uint32_t lane, Queue<K>& queue,
+                                         uint32_t& waiting, uint32_t& words)
+{
+  if constexpr (F < static_cast<int>(kQuickRun)) {
+    test_frustum<F, K>(run, item, t, rows, pair, lane, queue, waiting, words);
+    test_run<F + 1, K>(run, item, t, rows, pair, lane, queue, waiting, words);
+  }
+}
+
+// Tests a work item against its frusta, kQuickRun at a time, one mask word per
+// frustum and 64 objects.  Words that the quick test (quick_cull.hpp) decides whole
+// are stored together, a run's in one instruction; the others wait in the queue.
+// pair: the first run's entries of the item's list.  view_of(p0, p, frustum) gives
+// the lane the QuickView of the item's p-th frustum, in the run from p0 on; with
 // `last` the queue is drained before the return.
 template <int K, class ViewOf>
-__device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObjects<K>& t, uint32_t lane,
+__device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObjects<K>& t, KPair pair, uint32_t lane,
                                             const KPair* __restrict__ pairs, const SceneDev* __restrict__ scenes,
                                             const float* __restrict__ vps, unsigned long long* __restrict__ masks,
                                             Queue<K>& queue, uint32_t& waiting, uint32_t& words, bool last,
                                             ViewOf&& view_of)
 {
-  const KPair* const list = pairs + item.pair_begin;
-  uint32_t p = 0;
-  KPair next = list[0];  // (no item is made without pairs)
-  for (;;) {
-    bool full = false;
-    while (p < item.pair_count) {
-      const KPair q = next;
-      Mat16 m;
-      load_vp(vps, q.frustum, m);
-      const QuickView& view = view_of(p, q.frustum);
-      next = list[p + 1 < item.pair_count ? p + 1 : p];
-      unsigned long long bits[K], open[K];
-      uint32_t n_open = 0;
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const QuickResult<unsigned long long> r = quick_wave(t.quick[k], m.m, view);
-        bits[k] = (r.visible & t.tested[k]) | t.always[k];
-        open[k] = t.tested[k] & ~(r.visible | r.culled);
-        n_open += static_cast<uint32_t>(__builtin_popcountll(open[k]));
-      }
-      const uint64_t word = q.mask_word + item.tile_word;
-      if (n_open == 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-          // (a work item holds at least one object: the first word is always stored)
-          if (k == 0 || static_cast<uint32_t>(kWave * k) < item.count) masks[word + k] = bits[k];
-      } else {
-        full = waiting + n_open > Queue<K>::kCapacity;
-        if (full) {  // this frustum again, once the queue is empty
-          next = q;
-          break;
-        }
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          if (k != 0 && static_cast<uint32_t>(kWave * k) >= item.count) continue;
-          if (open[k] == 0) {
-            masks[word + k] = bits[k];
-            continue;
-          }
-          if ((open[k] >> lane) & 1) {
-            const uint64_t object = item.first_object + lane + kWave * k;
-            const uint32_t at = waiting + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(open[k] >> 32),
-                                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(open[k]), 0u));
-            queue.entry[at] = QueueEntry{static_cast<uint32_t>(object),
-                                         static_cast<uint32_t>(object >> 32) | (words << 16) | (lane << 24), q.frustum,
-                                         item.scene};
-          }
-          if (lane == 0) queue.word[words] = QueueWord{bits[k], word + k};
-          waiting += static_cast<uint32_t>(__builtin_popcountll(open[k]));
-          ++words;
-        }
-      }
-      ++p;
-    }
-    if (full | last) {
+  for (uint32_t p0 = 0;;) {
+    const uint32_t left = item.pair_count - p0, n = left < kQuickRun ? left : kQuickRun;
+    const QuickRows rows = quick_rows(view_of(p0, p0 + min(lane / 4 % kQuickRun, n - 1), pair.frustum), lane % 4);
+    const KPair next = load_pairs(pairs, item, p0 + kQuickRun, lane);
+    Run<K> run = {};
+    run.todo = (1u << n) - 1;
+    for (;;) {
+      test_run<0, K>(run, item, t, rows, pair, lane, queue, waiting, words);
+      if (run.again == 0) break;
       drain<K>(queue, waiting, words, lane, scenes, vps, masks);
       waiting = words = 0;
+      run.todo = run.again;
+      run.again = 0;
     }
-    if (!full) break;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      // (a work item holds at least one object: the first word is always stored)
+      if (k != 0 && static_cast<uint32_t>(kWave * k) >= item.count) break;
+      if (lane % 4 == 0 && lane / 4 < n && !((run.queued[k] >> (lane / 4)) & 1))
+        masks[pair.mask_word + item.tile_word + k] = static_cast<unsigned long long>(run.hi[k]) << 32 | run.lo[k];
+    }
+    if (left <= kQuickRun) break;
+    p0 += kQuickRun;
+    pair = next;
+  }
+  if (last) {
+    drain<K>(queue, waiting, words, lane, scenes, vps, masks);
+    waiting = words = 0;
   }
 }
 
-// Where a wave finds the QuickViews of its frusta: 38 vector instructions with
-// four square roots and 18 scalar ones would go into each use.  The batched kernel
-// keeps those of all frusta of a launch in LDS, computed once per workgroup (Table:
-// at most kTableViews frusta, 8 KB); without, and in the serving kernel, a wave
-// computes those of the list at hand, one per lane, kWave at a time.
+// Where a wave finds the QuickViews of its frusta: about a hundred instructions
+// with three square roots would go into each use.  The batched kernel keeps those
+// of all frusta of a launch in LDS, computed once per workgroup (Table: at most
+// kTableViews frusta, 12 KB); without, and in the serving kernel, a wave keeps those
+// of 64 frusta of its list, one per lane.
 constexpr uint32_t kTableViews = 128;
 constexpr uint32_t kBatchWaves = 4;  // waves of a workgroup, at most
 
@@ -252,8 +315,12 @@ __device__ __forceinline__ void list_views(const KPair* __restrict__ list, uint3
   wave_lds_order();
 }
 
+// The second launch bound keeps the 24 waves per CU of the default grid resident
+// (80 registers; at 95, and five waves per SIMD, 2,097,152 objects took 37.7 us
+// against 33.8), and has the matrix instructions' results in ordinary registers:
+// without one they are copied from the accumulation registers.
 template <int K, bool Table>
-__global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restrict__ items, uint32_t n_items,
+__global__ __launch_bounds__(256, K == 1 ? (Table ? 6 : 5) : K == 2 ? 4 : 2) void cull_batch_kernel(const WorkItem* __restrict__ items, uint32_t n_items,
                                                          const KPair* __restrict__ pairs,
                                                          const SceneDev* __restrict__ scenes,
                                                          const float* __restrict__ vps, uint32_t n_frusta,
@@ -272,6 +339,7 @@ __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restr
     Slot slot[K];
     RawObj raw[K];
     load_objects<K>(scenes, item, lane, slot, raw);
+    const KPair pair = load_pairs(pairs, item, 0, lane);
     if (first) {  // the table is built while the first objects are in flight
       if (Table) {
         for (uint32_t f = threadIdx.x; f < n_frusta; f += blockDim.x) {
@@ -286,12 +354,13 @@ __global__ __launch_bounds__(256) void cull_batch_kernel(const WorkItem* __restr
     TileObjects<K> objects;
     quick_objects<K>(slot, raw, objects);
     const bool last = it + n_waves >= n_items;
-    auto view_of = [&](uint32_t p, uint32_t f) -> const QuickView& {
+    auto view_of = [&](uint32_t p0, uint32_t p, uint32_t f) -> const QuickView& {
       if (Table) return table[f];
-      if (p % kWave == 0) list_views(pairs + item.pair_begin + p, item.pair_count - p, vps, lane, &table[wave * kWave]);
+      if (p0 % kWave == 0)
+        list_views(pairs + item.pair_begin + p0, item.pair_count - p0, vps, lane, &table[wave * kWave]);
       return table[wave * kWave + p % kWave];
     };
-    test_frusta<K>(item, objects, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, last, view_of);
+    test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, last, view_of);
     if (last) break;
     it += n_waves;
   }
@@ -328,7 +397,7 @@ __device__ __forceinline__ WorkItem serve_item(const ServeEntry& e, uint32_t til
 }
 
 template <int K>
-__global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __restrict__ entries, uint32_t n_entries,
+__global__ __launch_bounds__(256, 4) void cull_serve_kernel(const ServeEntry* __restrict__ entries, uint32_t n_entries,
                                                          uint64_t total_cost, const KPair* __restrict__ pairs,
                                                          const SceneDev* __restrict__ scenes,
                                                          const float* __restrict__ vps,
@@ -361,6 +430,7 @@ __global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __res
     Slot slot[K];
     RawObj raw[K];
     load_objects<K>(scenes, item, lane, slot, raw);
+    const KPair pair = load_pairs(pairs, item, 0, lane);
     if (viewed != a) {  // the entry's QuickViews, one per lane, while its first objects are in flight
       list_views(pairs + e.pair_begin, e.pair_count, vps, lane, views[block_wave]);
       viewed = a;
@@ -369,8 +439,8 @@ __global__ __launch_bounds__(256) void cull_serve_kernel(const ServeEntry* __res
     quick_objects<K>(slot, raw, objects);
     left -= count;
     const QuickView* const list = &views[block_wave][first];
-    test_frusta<K>(item, objects, lane, pairs, scenes, vps, masks, queues[block_wave], waiting, words, left == 0,
-                   [&](uint32_t p, uint32_t) -> const QuickView& { return list[p]; });
+    test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[block_wave], waiting, words, left == 0,
+                   [&](uint32_t, uint32_t p, uint32_t) -> const QuickView& { return list[p]; });
     if (left == 0) break;
     first = 0;
     for (++tile; tile >= e.tiles; tile = 0) e = entries[++a];  // (pairs are left: an entry with tiles follows)
@@ -486,35 +556,16 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   }
   for (size_t g = 0; g < n_groups; ++g) group_pair_begin[g + 1] += group_pair_begin[g];
 
-  if (!cfg) {
-    // Two objects per lane halve the per-frustum work that a wave does once for all
-    // its objects, and halve the waves: worth it where both are plenty (300,000
-    // objects x 32 views: 24.0 us against 25.7 with one; 1,000,000 x 8: 26.2
-    // against 25.5; 150,000 objects, 13,000 (tile, view) pairs: 9.9 against 8.8).
-    // The grid is then what the device holds at once, 16 waves per CU: with 24 the
-    // last third starts late (500,003 x 32: 36.4 us against 39.0).
-    uint64_t tiles = 0, tile_pairs = 0;
-    for (size_t g = 0; g < n_groups; ++g) {
-      const uint64_t n = group_pair_begin[g + 1] - group_pair_begin[g], t = (groups[g].count + kWave - 1) / kWave;
-      tiles += n ? t : 0;
-      tile_pairs += n * t;
-    }
-    if (tiles >= 16 * cus && tile_pairs >= 16 * tiles) {
-      c.objects_per_lane = 2;
-      c.waves_per_cu = 16;
-      plan->cfg = c;
-    }
-  }
   const uint64_t tile_objects = static_cast<uint64_t>(kWave) * c.objects_per_lane;
   if (c.max_frusta_per_item == 0) {
     // Where the tiles alone would leave the device idle, lists are split into
-    // slices of a length that gives about ten work items per CU (79 tiles x 64
-    // views: 15 us unsplit, 5.6 us in slices of 2, 5.9 of 1, 6.0 of 4; 625 tiles x
-    // 13 views: 6.6 us in slices of 4, 6.9 of 2, 7.4 of 8).  With eight tiles per
-    // CU a slice's second read of the objects costs more than it gives (2,344
-    // tiles x 6 views: 8.7 us unsplit, 9.9 in slices of 3); lists are then cut only
-    // after 16 views, so that the last items of a long launch are short (4,688
-    // tiles x 32 views: 25.5 us, 27 unsplit).
+    // slices of a length that gives about five work items per CU, of two views at
+    // least (79 tiles x 64 views: 10.3 us in slices of 32, 6.0 of 4, 6.3 of 2; 625 x
+    // 13: 6.8 us in slices of 16, 6.5 of 8, 6.8 of 4; 313 x 4: 5.2 us unsplit, 4.9 in
+    // slices of 2, 5.1 of 1).  With eight tiles per CU a slice's second read of the
+    // objects costs more than it gives (2,344 x 6: 7.6 us unsplit, 9.6 in slices of
+    // 4); lists are then cut only after 16 views, so that the last items of a long
+    // launch are short (1,563 x 64: 15.7 us in slices of 16, 16.2 of 32).
     uint64_t tiles = 0, tile_pairs = 0;
     for (size_t g = 0; g < n_groups; ++g) {
       const uint64_t n = group_pair_begin[g + 1] - group_pair_begin[g];
@@ -523,7 +574,7 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
       tile_pairs += n * t;
     }
     c.max_frusta_per_item =
-        tiles >= 8 * cus ? 16u : static_cast<uint32_t>(std::clamp<uint64_t>(tile_pairs / (10 * cus), 1, 16));
+        tiles >= 8 * cus ? 16u : static_cast<uint32_t>(std::clamp<uint64_t>((tile_pairs + 5 * cus - 1) / (5 * cus), 2, 16));
   }
   std::vector<WorkItem> items;
   for (size_t g = 0; g < n_groups; ++g) {
@@ -764,11 +815,13 @@ int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost,
   hipStream_t stream = as_stream(stream_handle);
   if (n_entries == 0 || total_cost == 0) return DPC_OK;
   const uint32_t waves_per_block = 4;
-  // A small batch is split into runs of a length that gives about ten waves per CU,
-  // as a batch plan's lists are (dpc_batch_plan_create).
+  // A small batch is split into runs of a length that gives about five waves per CU,
+  // as a batch plan's lists are (dpc_batch_plan_create); a large one into as many
+  // runs as the device holds waves (LDS: five workgroups per CU).
   const uint64_t cus = device_cu_count();
-  uint64_t waves = cus * (waves_per_cu ? waves_per_cu : 24);
-  waves = std::min(waves, total_cost / std::clamp<uint64_t>(total_cost / (10 * cus), 1, 16));
+  uint64_t waves = cus * (waves_per_cu ? waves_per_cu : 20);
+  waves = std::min(waves, total_cost / std::clamp<uint64_t>((total_cost + 5 * cus - 1) / (5 * cus), 2, 16));
+  if (waves == 0) waves = 1;
   const uint64_t blocks = (waves + waves_per_block - 1) / waves_per_block;
   const auto* e = static_cast<const ServeEntry*>(d_entries);
   const auto* p = static_cast<const KPair*>(d_pairs);

@@ -197,11 +197,38 @@ __device__ __forceinline__ bool obb_visible(const Obb& o, const float* vp)
 
 __device__ __forceinline__ QuickObj quick_of(const Obb& o) { return quick_obj(o.p, o.ex, o.ey, o.ez); }
 
-// The quick test of a wave's objects: lane masks.
-__device__ __forceinline__ QuickResult<unsigned long long> quick_wave(const QuickObj& q, const float* vp,
-                                                                      const QuickView& v)
+// What a wave holds of kQuickRun views: lane 4 f + i row i of view f, its norm, and
+// the view's factors of eps.
+constexpr uint32_t kQuickRun = 16;
+struct QuickRows {
+  float a[4], n, n3, n4;
+};
+__device__ __forceinline__ QuickRows quick_rows(const QuickView& v, uint32_t row)
 {
-  return quick_test<unsigned long long>(q, vp, v, [](float a, float b) { return ballot(a < b); });
+  return QuickRows{{v.a[row][0], v.a[row][1], v.a[row][2], v.a[row][3]}, v.n[row], v.n3, v.n4};
+}
+
+// The quick test of a wave's objects against view F of its rows: lane masks.  Four
+// outputs and four bounds per object are contractions over the object's centre and
+// over (s3, sw) and its radius, for 64 objects at once: 4x4x1 matrix instructions,
+// sixteen blocks of four objects, every block with the rows of view F (cbsz 4: one
+// block of the first operand for all sixteen; F is its number).  Each adds one
+// fused product per output, so a lane has its own object's outputs, bit for bit
+// those of quick_test.
+template <int F>
+__device__ __forceinline__ QuickResult<unsigned long long> quick_wave(const QuickObj& q, const QuickRows& v)
+{
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  const v4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  v4 out = __builtin_amdgcn_mfma_f32_4x4x1f32(v.a[0], q.cx, zero, 4, F, 0);
+  v4 bound = __builtin_amdgcn_mfma_f32_4x4x1f32(v.n, q.r, zero, 4, F, 0);
+  out = __builtin_amdgcn_mfma_f32_4x4x1f32(v.a[1], q.cy, out, 4, F, 0);
+  bound = __builtin_amdgcn_mfma_f32_4x4x1f32(v.n3, q.s3, bound, 4, F, 0);
+  out = __builtin_amdgcn_mfma_f32_4x4x1f32(v.a[2], q.cz, out, 4, F, 0);
+  bound = __builtin_amdgcn_mfma_f32_4x4x1f32(v.n4, q.sw, bound, 4, F, 0);
+  out = __builtin_amdgcn_mfma_f32_4x4x1f32(v.a[3], q.cw, out, 4, F, 0);
+  const float o[4] = {out.x, out.y, out.z, out.w}, b[4] = {bound.x, bound.y, bound.z, bound.w};
+  return quick_decide<unsigned long long>(o, b, [](float x, float y) { return ballot(x < y); });
 }
 
 // The raw inputs of one object as loaded from the SoA arrays: box (lower.xyz,

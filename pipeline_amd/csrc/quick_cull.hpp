@@ -8,18 +8,20 @@
 // where a corner lies within a rounding error of a plane.  Everywhere else any
 // evaluation with a known error bound gives the same answer: here the clip-space
 // centre of the object (twice the centre, 2p + ex + ey + ez) and a sphere around
-// it, 38 operations with fused multiply-adds.  A pair closer to a plane than
-// `eps`, a bound on all rounding errors of both evaluations, is left undecided, and
-// so is one whose sphere reaches a plane that its centre lies outside of: 2 to 10
-// in a thousand of the pairs of ordinary scenes, most of which do touch a plane.
+// it: 28 fused multiply-adds, which run on the matrix cores, and 11 operations
+// more.  A pair closer to a plane than `eps`, a bound on all rounding errors of both
+// evaluations, is left undecided, and so is one whose sphere reaches a plane that
+// its centre lies outside of: 2 to 10 in a thousand of the pairs of ordinary
+// scenes, most of which do touch a plane.
 //
 // In terms of the exact sums over the eight corners, with w and c (= x, y or z)
 // the clip coordinates, the reference reports an object culled when on some axis
 // all corners have c <= -w, or all have w <= c and none has c <= -w.
 //   visible   the centre lies inside all six planes: some corner then lies
 //             strictly inside each of them
-//   culled    x, y: |c| - |w| > r max(|Mw - Mc|, |Mw + Mc|) at the centre: every
-//             corner is beyond the same plane, and (for c > 0) none has c <= -w
+//   culled    x, y: max(|x|, |y|) - |w| > r n, n the largest of |Mw - Mx|, |Mw + Mx|,
+//             |Mw - My|, |Mw + My|, at the centre: every corner is beyond the same
+//             plane, and (for c > 0) none has c <= -w
 //             z: every corner has z < -w; or every corner has w < z and z > -w
 // (Mc: the first three elements of a column of the matrix; r: the sphere's radius.)
 // z uses the sums z + w and w - z of the matrix's columns: for a distant far
@@ -34,15 +36,18 @@
 // The bound.  u = 2^-24, A_j = |p_j| + |ex_j| + |ey_j| + |ez_j|, S_c = sum_j A_j
 // |M_jc|, everything in the doubled scale.  Errors of the exact test's corners:
 // 14 u S_c per coordinate (four-term products 4 u, three adds 3 u, doubled).
-// Errors here: centre 12 u S_c per coordinate, or 14 u (S_z + S_w) by the column
-// sums, and 4 u (S_c + S_w) of the last adds: 30 u (S_c + S_w) together.  S_c + S_w
-// <= 2 (n3 * s3 + n4 * sw) with n3, n4 the largest magnitudes of rows 0-2 and row 3,
-// s3 >= sum of A_j over x, y, z (the edges' part is at most 3 r), sw = A_w; the
-// differences of columns inside the norms lose at most 12 u n3 s3 more.  eps = 2^-17
-// (n3 s3 + n4 sw) = 128 u (n3 s3 + n4 sw) against those 72.  The added 2^-117 and
-// 2^-130 cover underflow.  Operands of 2^56 (matrix) or 2^60 (object) and above,
-// infinities and NaN make eps infinite or NaN, and every comparison below false:
-// undecided.  So does an object whose edges have a w component.
+// Errors here: centre 12 u S_c per coordinate, 14 u (S_z + S_w) for each of z + w
+// and w - z and so twice that for their sum, and 3 u (S_c + S_w) of the last adds.
+// S_c <= T = n3 s3 + n4 sw with n3, n4 the largest magnitudes of rows 0-2 and row 3,
+// s3 >= sum of A_j over x, y, z (the edges' part is at most 3 r), sw = A_w.  The
+// differences of columns inside the norms lose at most 12 u T more.  The tests of x
+// and y are made at twice that scale: 2 (28 + 12 + 28 + 5 + 12) u T = 170 u T at most,
+// those of z + w and w - z at once that scale: 90 u T.  eps = 2^-16 (n3 s3 + n4 sw) =
+// 256 u T serves both.  The 2^-90 and 2^-117 added to the object's factors cover
+// underflow.  Operands of 2^56 (matrix) or 2^60 (object) and above, matrices whose
+// rows 0-2 lie below 2^-47, infinities and NaN make eps infinite or NaN, and every
+// comparison below false: undecided.  So does an object whose edges have a w
+// component.
 #pragma once
 
 #include <cstdint>
@@ -62,11 +67,14 @@ struct QuickObj {
   float s3, sw;          // the object's factors of eps
 };
 
-// What it reads of a view-projection matrix beside its elements.
+// What it reads of a view-projection matrix: rows of four clip-space outputs of the
+// centre, all at twice their scale, 2x, 2y, z + w and w - z (whose sum is 2w), and
+// of the bounds that go with them: r n[i] + eps, with the norms of w - x, w + x,
+// w - y and w + y (the largest, doubled), of z + w, of w - z, and 0.
 struct alignas(16) QuickView {
-  float lo[4], hi[4];    // rows of z + w and w - z
-  float nx, ny, nl, nh;  // norms: of w - x or w + x, of w - y or w + y (the larger), of z + w, of w - z
-  float n3, n4;          // largest magnitude in rows 0-2, in row 3 (infinite from 2^56 on)
+  float a[4][4];
+  float n[4];
+  float n3, n4;  // twice the largest magnitude in rows 0-2, in row 3 (infinite: decides nothing)
   float pad[2];
 };
 
@@ -107,7 +115,7 @@ DPC_HD QuickObj quick_obj(const V4& p, const V4& ex, const V4& ey, const V4& ez)
   const float aw = __builtin_fabsf(p.w);
   const float a3 = quick_fma(3.0f, q.r, (__builtin_fabsf(p.x) + __builtin_fabsf(p.y)) + __builtin_fabsf(p.z));
   const bool fits = (flat == 0.0f) & (a3 + aw < 0x1p60f);  // (false for NaN)
-  q.s3 = fits ? quick_fma(a3, 0x1p-17f, 0x1p-117f) : __builtin_inff();
+  q.s3 = fits ? quick_fma(a3, 0x1p-17f, 0x1p-90f) : __builtin_inff();
   q.sw = quick_fma(aw, 0x1p-17f, 0x1p-117f);
   return q;
 }
@@ -117,30 +125,27 @@ DPC_HD QuickObj quick_obj(const V4& p, const V4& ex, const V4& ey, const V4& ez)
 // which run on the scalar unit for a wave-uniform matrix).
 DPC_HD uint32_t quick_magnitude(float v) { return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu; }
 
-// (2^56 and above: infinite)
-DPC_HD float quick_scale(uint32_t bits)
-{
-  return __builtin_bit_cast(float, bits >= 0x5b800000u ? 0x7f800000u : bits);
-}
-
 DPC_HD QuickView quick_view(const float* m)
 {
   QuickView v;
   for (int j = 0; j < 4; ++j) {
-    v.lo[j] = m[4 * j + 2] + m[4 * j + 3];
-    v.hi[j] = m[4 * j + 3] - m[4 * j + 2];
+    v.a[0][j] = 2.0f * m[4 * j];
+    v.a[1][j] = 2.0f * m[4 * j + 1];
+    v.a[2][j] = m[4 * j + 2] + m[4 * j + 3];
+    v.a[3][j] = m[4 * j + 3] - m[4 * j + 2];
   }
-  v.nl = quick_root(quick_dot(v.lo[0], v.lo[1], v.lo[2], v.lo[0], v.lo[1], v.lo[2]));
-  v.nh = quick_root(quick_dot(v.hi[0], v.hi[1], v.hi[2], v.hi[0], v.hi[1], v.hi[2]));
-  float n[2];
+  float n = 0.0f;  // the largest of w - x, w + x, w - y, w + y, squared (NaN: n3 is NaN too)
   for (int c = 0; c < 2; ++c) {
     const float d0 = m[3] - m[c], d1 = m[7] - m[4 + c], d2 = m[11] - m[8 + c];
     const float s0 = m[3] + m[c], s1 = m[7] + m[4 + c], s2 = m[11] + m[8 + c];
     const float d = quick_dot(d0, d1, d2, d0, d1, d2), s = quick_dot(s0, s1, s2, s0, s1, s2);
-    n[c] = quick_root(d > s ? d : s);  // (NaN: n3 is NaN too)
+    n = d > n ? d : n;
+    n = s > n ? s : n;
   }
-  v.nx = n[0];
-  v.ny = n[1];
+  v.n[0] = 2.0f * quick_root(n);
+  for (int i = 2; i < 4; ++i)
+    v.n[i - 1] = quick_root(quick_dot(v.a[i][0], v.a[i][1], v.a[i][2], v.a[i][0], v.a[i][1], v.a[i][2]));
+  v.n[3] = 0.0f;
   uint32_t n3 = 0, n4 = 0;
   for (int k = 0; k < 12; ++k) {
     const uint32_t b = quick_magnitude(m[k]);
@@ -150,8 +155,9 @@ DPC_HD QuickView quick_view(const float* m)
     const uint32_t b = quick_magnitude(m[k]);
     n4 = b > n4 ? b : n4;
   }
-  v.n3 = quick_scale(n3);
-  v.n4 = quick_scale(n4);
+  // (2^56 and above, and below 2^-47, where 2^-90 n3 would not cover underflow)
+  v.n3 = n3 >= 0x5b800000u || n3 < 0x28000000u ? __builtin_inff() : 2.0f * __builtin_bit_cast(float, n3);
+  v.n4 = n4 >= 0x5b800000u ? __builtin_inff() : 2.0f * __builtin_bit_cast(float, n4);
   v.pad[0] = v.pad[1] = 0.0f;
   return v;
 }
@@ -166,23 +172,38 @@ struct QuickResult {
   M culled;   // certainly culled (neither: undecided)
 };
 
+// out: the view's four outputs at the object's centre; bound: r n[i] + eps.
 template <class M, class Less>
-DPC_HD QuickResult<M> quick_test(const QuickObj& q, const float* m, const QuickView& v, Less&& less)
+DPC_HD QuickResult<M> quick_decide(const float (&out)[4], const float (&bound)[4], Less&& less)
 {
-  const float eps = quick_fma(v.n3, q.s3, quick_fma(v.n4, q.sw, 0x1p-130f));
-  // clip-space centre: x, y, w from the matrix, z + w and w - z from its column sums
-  const float cx = quick_fma(q.cw, m[12], quick_fma(q.cz, m[8], quick_fma(q.cy, m[4], q.cx * m[0])));
-  const float cy = quick_fma(q.cw, m[13], quick_fma(q.cz, m[9], quick_fma(q.cy, m[5], q.cx * m[1])));
-  const float cw = quick_fma(q.cw, m[15], quick_fma(q.cz, m[11], quick_fma(q.cy, m[7], q.cx * m[3])));
-  const float dl = quick_fma(q.cw, v.lo[3], quick_fma(q.cz, v.lo[2], quick_fma(q.cy, v.lo[1], q.cx * v.lo[0])));
-  const float dh = quick_fma(q.cw, v.hi[3], quick_fma(q.cz, v.hi[2], quick_fma(q.cy, v.hi[1], q.cx * v.hi[0])));
-  const float acx = __builtin_fabsf(cx), acy = __builtin_fabsf(cy);
-  const float inner = cw - eps, outer = __builtin_fabsf(cw) + eps;
+  const float ax = __builtin_fabsf(out[0]), ay = __builtin_fabsf(out[1]), l = out[2], h = out[3], eps = bound[3];
+#ifdef __HIP_DEVICE_COMPILE__
+  // (the median with an infinity that the compiler does not see: one instruction,
+  // where a maximum first quiets its operands)
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  const float far = __builtin_amdgcn_fmed3f(ax, ay, inf), near = __builtin_amdgcn_fmed3f(l, h, -inf);
+#else
+  const float far = ax < ay ? ay : ax, near = l < h ? l : h;
+#endif
+  const float w = l + h;
   QuickResult<M> r;
-  r.visible = less(acx, inner) & less(acy, inner) & less(eps, dl) & less(eps, dh);
-  r.culled = less(quick_fma(q.r, v.nx, outer), acx) | less(quick_fma(q.r, v.ny, outer), acy) |
-             less(quick_fma(q.r, v.nl, dl), -eps) | (less(quick_fma(q.r, v.nh, dh), -eps) & less(eps, quick_fma(-q.r, v.nl, dl)));
+  r.visible = less(far, w - eps) & less(eps, near);
+  r.culled = less(__builtin_fabsf(w) + bound[0], far) | less(bound[1], -l) | (less(bound[2], -h) & less(bound[1], l));
   return r;
+}
+
+// The outputs and bounds of one object and view.  The device computes them with
+// matrix instructions that add one product after the other, fused, in this order.
+template <class M, class Less>
+DPC_HD QuickResult<M> quick_test(const QuickObj& q, const QuickView& v, Less&& less)
+{
+  float out[4], bound[4];
+  for (int i = 0; i < 4; ++i) {
+    out[i] = quick_fma(q.cw, v.a[i][3], quick_fma(q.cz, v.a[i][2], quick_fma(q.cy, v.a[i][1], q.cx * v.a[i][0])));
+    bound[i] = quick_fma(q.sw, v.n4, quick_fma(q.s3, v.n3, q.r * v.n[i]));
+  }
+  return quick_decide<M>(out, bound, less);
 }
 
 }  // namespace dpc

@@ -89,7 +89,7 @@ void check(const float obb[16], const float vp[16], const char* what)
   std::memcpy(v, obb, sizeof v);
   const dpc::QuickObj q = dpc::quick_obj(v[0], v[1], v[2], v[3]);
   const dpc::QuickView view = dpc::quick_view(vp);
-  const auto r = dpc::quick_test<bool>(q, vp, view, [](float a, float b) { return a < b; });
+  const auto r = dpc::quick_test<bool>(q, view, [](float a, float b) { return a < b; });
   const bool want = orc_is_visible_obb(vp, obb) != 0;
   ++pairs;
   if (r.visible || r.culled) ++decided;

@@ -49,7 +49,9 @@ def oracle_masks(lower, upper, mats, xform, vps):
 @pytest.mark.parametrize("n,frusta,cfg", [
     (1, 1, None), (63, 3, None), (64, 128, None), (65, 129, None), (4_097, 17, None), (40_001, 33, None),
     (4_097, 70, (1, 256, 1, 70)), (4_097, 129, (2, 64, 4, 0)), (1_000, 40, (2, 256, 2, 40)), (1_025, 130, (4, 128, 1, 130)),
-    (5_000, 20, (4, 256, 8, 3))])
+    (5_000, 20, (4, 256, 8, 3)),
+    (4_097, 15, None), (4_097, 16, (1, 256, 24, 64)), (1_000, 31, (2, 256, 16, 64)), (1_000, 32, (4, 256, 8, 64)),
+    (200, 144, (1, 256, 24, 144))])
 def test_batch_masks(n, frusta, cfg, undecided):
     rng = np.random.default_rng(n + frusta)
     lower, upper, mats, xform = make_scene(n, undecided, n)
