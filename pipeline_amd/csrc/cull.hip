@@ -68,6 +68,44 @@ __global__ __launch_bounds__(Indexed ? kIndexedThreads : kPlainThreads) void cul
   }
 }
 
+// The same, two adjacent tiles per wave (launch_cull: where): both tiles' indices,
+// then both tiles' boxes and rows are in flight together, and half as many waves
+// start and end.
+constexpr unsigned kPairThreads = 256;
+
+template <bool Diff>
+__global__ __launch_bounds__(kPairThreads) void cull_pair_kernel(const float4* __restrict__ box_a,
+                                                                 const float2* __restrict__ box_b,
+                                                                 const uint32_t* __restrict__ xform, size_t n,
+                                                                 const float4* __restrict__ planes, size_t ld, Mat16 vp,
+                                                                 unsigned long long* __restrict__ mask,
+                                                                 const unsigned long long* __restrict__ old,
+                                                                 uint8_t* __restrict__ count)
+{
+  const unsigned lane = threadIdx.x & (kWave - 1);
+  const size_t first = (static_cast<size_t>(blockIdx.x) * kPairThreads + (threadIdx.x & ~(kWave - 1u))) * 2 + lane;
+  Slot s[2];
+  RawObj r[2];
+  unsigned long long old_bits[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const size_t i = first + kWave * k;
+    old_bits[k] = Diff && lane == 0 && i < n ? old[i >> 6] : 0ull;
+    s[k] = make_slot(i, n, xform, ld);
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) r[k] = load_raw(box_a, box_b, planes, ld, s[k].i, s[k].m);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const size_t i = first + kWave * k;
+    const unsigned long long bits = __ballot(slot_visible(s[k], obb_visible(obb_of(r[k]), vp.m)));
+    if (lane == 0 && i < n) {
+      mask[i >> 6] = bits;
+      if (Diff) count[i >> 6] = changed_in_word(old_bits[k], bits, i >> 6, n);
+    }
+  }
+}
+
 // Streaming form: a persistent grid in which every wave walks tiles t, t+W,
 // t+2W, ... with two register sets: while one tile is tested, the loads of the
 // next one are in flight.  Every wave runs the same number of steps (tiles past
@@ -969,7 +1007,17 @@ int launch_cull(const float* d_box_a, const float* d_box_b, const uint32_t* d_xf
   const size_t tiles = (n_objects + kWave - 1) / kWave;
   hipStream_t s = as_stream(stream);
   if (cfg.waves_per_cu == 0) {
-    if (d_xform)
+    // Two tiles per wave where three objects or more share a matrix and the call is
+    // long: a tile then reads 40 to 45 bytes an object and waits for latency more than
+    // for memory (2,372,871 objects with 4 to a matrix: 19.9 -> 18.5 us; 4,900,000:
+    // 44.1 -> 39.2, with 7 41.6 -> 35.8; 1,500,000 with 4: 13.0 -> 12.7).  Shorter
+    // calls lose by the waves they no longer have (700,000 with 4: 8.2 -> 8.4 us;
+    // 400,000: 5.8 -> 6.3), and with a matrix to each object or two memory is the
+    // bound (4,900,000: 72.8 -> 75.2 with one, 50.4 -> 50.8 with two).
+    if (d_xform && n_objects >= 1'400'000 && n_objects / 3 >= ld)
+      hipLaunchKernelGGL((cull_pair_kernel<Diff>), dim3(grid_for((n_objects + 1) / 2, kPairThreads)), dim3(kPairThreads), 0,
+                         s, a, b, d_xform, n_objects, p, ld, m, out, old, count);
+    else if (d_xform)
       hipLaunchKernelGGL((cull_kernel<true, Diff>), dim3(grid_for(n_objects, kIndexedThreads)), dim3(kIndexedThreads), 0, s,
                          a, b, d_xform, n_objects, p, ld, m, out, old, count);
     else
