@@ -197,15 +197,15 @@ __device__ __forceinline__ bool obb_visible(const Obb& o, const float* vp)
 
 __device__ __forceinline__ QuickObj quick_of(const Obb& o) { return quick_obj(o.p, o.ex, o.ey, o.ez); }
 
-// What a wave holds of kQuickRun views: lane 4 f + i row i of view f, its norm, and
-// the view's factors of eps.
+// What a wave holds of kQuickRun views: lane 4 f + i row i of view f, its norm and
+// its factors of eps.
 constexpr uint32_t kQuickRun = 16;
 struct QuickRows {
   float a[4], n, n3, n4;
 };
 __device__ __forceinline__ QuickRows quick_rows(const QuickView& v, uint32_t row)
 {
-  return QuickRows{{v.a[row][0], v.a[row][1], v.a[row][2], v.a[row][3]}, v.n[row], v.n3, v.n4};
+  return QuickRows{{v.a[row][0], v.a[row][1], v.a[row][2], v.a[row][3]}, v.n[row], v.n34[row / 2][0], v.n34[row / 2][1]};
 }
 
 // The quick test of a wave's objects against view F of its rows: lane masks.  Four

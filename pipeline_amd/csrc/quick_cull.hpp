@@ -8,7 +8,7 @@
 // where a corner lies within a rounding error of a plane.  Everywhere else any
 // evaluation with a known error bound gives the same answer: here the clip-space
 // centre of the object (twice the centre, 2p + ex + ey + ez) and a sphere around
-// it: 28 fused multiply-adds, which run on the matrix cores, and 11 operations
+// it: 28 fused multiply-adds, which run on the matrix cores, and 14 operations
 // more.  A pair closer to a plane than `eps`, a bound on all rounding errors of both
 // evaluations, is left undecided, and so is one whose sphere reaches a plane that
 // its centre lies outside of: 2 to 10 in a thousand of the pairs of ordinary
@@ -19,9 +19,8 @@
 // all corners have c <= -w, or all have w <= c and none has c <= -w.
 //   visible   the centre lies inside all six planes: some corner then lies
 //             strictly inside each of them
-//   culled    x, y: max(|x|, |y|) - |w| > r n, n the largest of |Mw - Mx|, |Mw + Mx|,
-//             |Mw - My|, |Mw + My|, at the centre: every corner is beyond the same
-//             plane, and (for c > 0) none has c <= -w
+//   culled    x, y: |c| - |w| > r max(|Mw - Mc|, |Mw + Mc|) at the centre: every
+//             corner is beyond the same plane, and (for c > 0) none has c <= -w
 //             z: every corner has z < -w; or every corner has w < z and z > -w
 // (Mc: the first three elements of a column of the matrix; r: the sphere's radius.)
 // z uses the sums z + w and w - z of the matrix's columns: for a distant far
@@ -34,20 +33,22 @@
 // than the underflow of squares hides.
 //
 // The bound.  u = 2^-24, A_j = |p_j| + |ex_j| + |ey_j| + |ez_j|, S_c = sum_j A_j
-// |M_jc|, everything in the doubled scale.  Errors of the exact test's corners:
-// 14 u S_c per coordinate (four-term products 4 u, three adds 3 u, doubled).
-// Errors here: centre 12 u S_c per coordinate, 14 u (S_z + S_w) for each of z + w
-// and w - z and so twice that for their sum, and 3 u (S_c + S_w) of the last adds.
-// S_c <= T = n3 s3 + n4 sw with n3, n4 the largest magnitudes of rows 0-2 and row 3,
-// s3 >= sum of A_j over x, y, z (the edges' part is at most 3 r), sw = A_w.  The
-// differences of columns inside the norms lose at most 12 u T more.  The tests of x
-// and y are made at twice that scale: 2 (28 + 12 + 28 + 5 + 12) u T = 170 u T at most,
-// those of z + w and w - z at once that scale: 90 u T.  eps = 2^-16 (n3 s3 + n4 sw) =
-// 256 u T serves both.  The 2^-90 and 2^-117 added to the object's factors cover
-// underflow.  Operands of 2^56 (matrix) or 2^60 (object) and above, matrices whose
-// rows 0-2 lie below 2^-47, infinities and NaN make eps infinite or NaN, and every
-// comparison below false: undecided.  So does an object whose edges have a w
-// component.
+// |M_jc|, everything in the doubled scale.  S_c <= T = n3 s3 + n4 sw with n3, n4 the
+// largest magnitudes of rows 0-2 and row 3, s3 >= sum of A_j over x, y, z (the
+// edges' part is at most 3 r), sw = A_w.  Errors of the exact test's corners: 14 u
+// S_c per coordinate (four-term products 4 u, three adds 3 u, doubled).  Errors
+// here: the centre 3 u A_j and the products 8 u, 11 u S_c per coordinate; the sums
+// and differences of columns 2 u more, 13 u (S_z + S_w) <= 26 u T for each of z + w
+// and w - z.  What the norms lose before they are rounded up is below 2 u T.
+//   z + w, w - z       28 + 26 + 2 = 56 u T
+//   x and w, at twice the scale: 2 (14 u S_x + 14 u S_w) <= 56, x 22, w 52, the last
+//   two adds 8, the norms 4: 142 u T, and 138 without the norms
+// The bounds take 80 u T for z + w and w - z and 160 u T for x and y, and the tests
+// for `visible` 80 and twice that: 2^-17 s3 and 2^-17 sw (128 u) times 0.625 and 1.25
+// of n3 and n4.  The 2^-90 and 2^-117 added to the object's factors cover underflow.
+// Operands of 2^56 (matrix) or 2^60 (object) and above, matrices whose rows 0-2 lie
+// below 2^-47, infinities and NaN make eps infinite or NaN, and every comparison
+// below false: undecided.  So does an object whose edges have a w component.
 #pragma once
 
 #include <cstdint>
@@ -69,13 +70,14 @@ struct QuickObj {
 
 // What it reads of a view-projection matrix: rows of four clip-space outputs of the
 // centre, all at twice their scale, 2x, 2y, z + w and w - z (whose sum is 2w), and
-// of the bounds that go with them: r n[i] + eps, with the norms of w - x, w + x,
-// w - y and w + y (the largest, doubled), of z + w, of w - z, and 0.
+// the norms of their bounds, r n[i] + eps: of w - x or w + x (the larger, doubled),
+// of w - y or w + y, of z + w and of w - z.  n3, n4: the largest magnitudes in rows
+// 0-2 and in row 3 as factors of eps, [0] for x and y, [1] for z + w and w - z
+// (infinite: decides nothing).
 struct alignas(16) QuickView {
   float a[4][4];
   float n[4];
-  float n3, n4;  // twice the largest magnitude in rows 0-2, in row 3 (infinite: decides nothing)
-  float pad[2];
+  float n34[2][2];  // [0]: n3, n4 for x and y
 };
 
 DPC_HD float quick_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -134,18 +136,14 @@ DPC_HD QuickView quick_view(const float* m)
     v.a[2][j] = m[4 * j + 2] + m[4 * j + 3];
     v.a[3][j] = m[4 * j + 3] - m[4 * j + 2];
   }
-  float n = 0.0f;  // the largest of w - x, w + x, w - y, w + y, squared (NaN: n3 is NaN too)
   for (int c = 0; c < 2; ++c) {
     const float d0 = m[3] - m[c], d1 = m[7] - m[4 + c], d2 = m[11] - m[8 + c];
     const float s0 = m[3] + m[c], s1 = m[7] + m[4 + c], s2 = m[11] + m[8 + c];
     const float d = quick_dot(d0, d1, d2, d0, d1, d2), s = quick_dot(s0, s1, s2, s0, s1, s2);
-    n = d > n ? d : n;
-    n = s > n ? s : n;
+    v.n[c] = 2.0f * quick_root(d > s ? d : s);  // (NaN: n3 is NaN too)
   }
-  v.n[0] = 2.0f * quick_root(n);
   for (int i = 2; i < 4; ++i)
-    v.n[i - 1] = quick_root(quick_dot(v.a[i][0], v.a[i][1], v.a[i][2], v.a[i][0], v.a[i][1], v.a[i][2]));
-  v.n[3] = 0.0f;
+    v.n[i] = quick_root(quick_dot(v.a[i][0], v.a[i][1], v.a[i][2], v.a[i][0], v.a[i][1], v.a[i][2]));
   uint32_t n3 = 0, n4 = 0;
   for (int k = 0; k < 12; ++k) {
     const uint32_t b = quick_magnitude(m[k]);
@@ -156,9 +154,12 @@ DPC_HD QuickView quick_view(const float* m)
     n4 = b > n4 ? b : n4;
   }
   // (2^56 and above, and below 2^-47, where 2^-90 n3 would not cover underflow)
-  v.n3 = n3 >= 0x5b800000u || n3 < 0x28000000u ? __builtin_inff() : 2.0f * __builtin_bit_cast(float, n3);
-  v.n4 = n4 >= 0x5b800000u ? __builtin_inff() : 2.0f * __builtin_bit_cast(float, n4);
-  v.pad[0] = v.pad[1] = 0.0f;
+  const float f3 = n3 >= 0x5b800000u || n3 < 0x28000000u ? __builtin_inff() : __builtin_bit_cast(float, n3);
+  const float f4 = n4 >= 0x5b800000u ? __builtin_inff() : __builtin_bit_cast(float, n4);
+  v.n34[0][0] = 1.25f * f3;
+  v.n34[0][1] = 1.25f * f4;
+  v.n34[1][0] = 0.625f * f3;
+  v.n34[1][1] = 0.625f * f4;
   return v;
 }
 
@@ -172,24 +173,28 @@ struct QuickResult {
   M culled;   // certainly culled (neither: undecided)
 };
 
-// out: the view's four outputs at the object's centre; bound: r n[i] + eps.
+// out: the view's four outputs at the object's centre; bound: r n[i] + eps.  For
+// `visible`, in place of eps itself the smaller bound of z + w and w - z serves: of
+// one of them the norm is small wherever near and far plane lie apart.
 template <class M, class Less>
 DPC_HD QuickResult<M> quick_decide(const float (&out)[4], const float (&bound)[4], Less&& less)
 {
-  const float ax = __builtin_fabsf(out[0]), ay = __builtin_fabsf(out[1]), l = out[2], h = out[3], eps = bound[3];
+  const float ax = __builtin_fabsf(out[0]), ay = __builtin_fabsf(out[1]), l = out[2], h = out[3];
 #ifdef __HIP_DEVICE_COMPILE__
   // (the median with an infinity that the compiler does not see: one instruction,
   // where a maximum first quiets its operands)
   float inf = __builtin_inff();
   asm("" : "+s"(inf));
   const float far = __builtin_amdgcn_fmed3f(ax, ay, inf), near = __builtin_amdgcn_fmed3f(l, h, -inf);
+  const float eps = __builtin_amdgcn_fmed3f(bound[2], bound[3], -inf);
 #else
-  const float far = ax < ay ? ay : ax, near = l < h ? l : h;
+  const float far = ax < ay ? ay : ax, near = l < h ? l : h, eps = bound[2] < bound[3] ? bound[2] : bound[3];
 #endif
-  const float w = l + h;
+  const float w = l + h, aw = __builtin_fabsf(w);
   QuickResult<M> r;
-  r.visible = less(far, w - eps) & less(eps, near);
-  r.culled = less(__builtin_fabsf(w) + bound[0], far) | less(bound[1], -l) | (less(bound[2], -h) & less(bound[1], l));
+  r.visible = less(far, quick_fma(-2.0f, eps, w)) & less(eps, near);
+  r.culled = less(aw + bound[0], ax) | less(aw + bound[1], ay) | less(bound[2], -l) |
+             (less(bound[3], -h) & less(bound[2], l));
   return r;
 }
 
@@ -201,7 +206,7 @@ DPC_HD QuickResult<M> quick_test(const QuickObj& q, const QuickView& v, Less&& l
   float out[4], bound[4];
   for (int i = 0; i < 4; ++i) {
     out[i] = quick_fma(q.cw, v.a[i][3], quick_fma(q.cz, v.a[i][2], quick_fma(q.cy, v.a[i][1], q.cx * v.a[i][0])));
-    bound[i] = quick_fma(q.sw, v.n4, quick_fma(q.s3, v.n3, q.r * v.n[i]));
+    bound[i] = quick_fma(q.sw, v.n34[i / 2][1], quick_fma(q.s3, v.n34[i / 2][0], q.r * v.n[i]));
   }
   return quick_decide<M>(out, bound, less);
 }
