@@ -318,7 +318,7 @@ int dpc_bbox(const float* d_box_a, const float* d_box_b, const uint32_t* d_xform
  * scenes (a quarter of the budget, at most 1 GiB, is the in-flight arena,
  * split over streams x batches_per_stream batches).  Each batch also has a
  * pinned host arena of the same size, at most 32 MiB, where its descriptors and
- * copied deltas are gathered for one transfer. */
+ * deltas are gathered for one transfer. */
 typedef struct dpc_server dpc_server;
 
 typedef struct dpc_server_config {
@@ -330,7 +330,7 @@ typedef struct dpc_server_config {
   uint32_t batches_per_stream;  /* batches in flight per stream (0: 2, at most 4) */
   uint32_t direct_delta_reads;  /* 1: a delta whose two arrays each lie in one pinned host
                                    allocation is read by the device directly, with no
-                                   copy; 0: every delta is copied to the device first */
+                                   copy; 0: every delta goes through the batch's arena */
   uint64_t hbm_budget_bytes;    /* resident scenes + in-flight requests */
 } dpc_server_config;
 

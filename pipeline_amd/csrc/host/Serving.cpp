@@ -9,11 +9,11 @@
 // scene, until the arena is full.  A scene with requests in flight is bound to
 // the stream that runs them and joins only batches of that stream: stream order
 // then keeps each scene's requests in submission order (each sees the deltas
-// of the earlier ones) without waiting for them to finish.  A batch copies the
-// deltas to the device (gathered on the host into one copy, each matrix as its
-// first three columns when the batch's last columns are all 0 0 0 1) and
-// scatters them into the scenes' matrices, tests every
-// scene of the batch against its request's frusta in one launch
+// of the earlier ones) without waiting for them to finish.  A batch's deltas are
+// gathered in its pinned arena (each matrix as its first three columns when the
+// delta's last columns are all 0 0 0 1) and scattered into the scenes' matrices by
+// one launch, which reads the arena itself or, when they are many, the copy of it
+// made first.  The batch then tests every scene of the batch against its request's frusta in one launch
 // (dpc::launch_serve), then copies each request's masks to its caller's
 // buffer.  Batches on different streams overlap on the device.
 //
@@ -53,7 +53,7 @@ constexpr uint32_t kMaxFrusta = 64;
 // the pinned staging area of one batch's descriptors (entries, pairs, frusta, copy-outs)
 constexpr uint64_t kHostArena = 4096 + kMaxBatch * 32 + kMaxBatch * kMaxFrusta * (16 + 64) + kMaxBatch * 32 + 4 * 256;
 // ... which also stages the batch's deltas when they fit: the batch then
-// crosses PCIe in one copy instead of two per request
+// crosses PCIe once instead of in two copies per request
 constexpr uint64_t kHostStageMax = 32ull << 20;
 // a delta's matrices up to this size are staged; a larger array is copied on its own
 constexpr uint64_t kStageMatsMax = kHostStageMax;
