@@ -13,8 +13,8 @@
 // gathered in its pinned arena (each matrix as its first three columns when the
 // delta's last columns are all 0 0 0 1) and scattered into the scenes' matrices by
 // one launch, which reads the arena itself or, when they are many, the copy of it
-// made first.  The batch then tests every scene of the batch against its request's frusta in one launch
-// (dpc::launch_serve), then copies each request's masks to its caller's
+// made first.  The batch then tests every scene against its request's frusta in one
+// launch (dpc::launch_serve) and copies each request's masks to its caller's
 // buffer.  Batches on different streams overlap on the device.
 //
 // The HIP calls of a batch are made by its stream's issuer thread, one per
