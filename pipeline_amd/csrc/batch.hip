@@ -597,12 +597,14 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
       }
     }
   }
-  // Largest items first (cost = frusta x 64-object words).
-  std::stable_sort(items.begin(), items.end(), [](const WorkItem& a, const WorkItem& b) {
+  // Largest items first (cost = frusta x 64-object words); lists of one length are
+  // in that order already.
+  const auto larger = [](const WorkItem& a, const WorkItem& b) {
     const uint64_t ca = static_cast<uint64_t>(a.pair_count) * ((a.count + 63) / 64);
     const uint64_t cb = static_cast<uint64_t>(b.pair_count) * ((b.count + 63) / 64);
     return ca > cb;
-  });
+  };
+  if (!std::is_sorted(items.begin(), items.end(), larger)) std::stable_sort(items.begin(), items.end(), larger);
   if (items.size() > 0xFFFFFFFFull) {
     free_plan(plan);
     return set_error(DPC_ERR_INVALID_ARGUMENT, "dpc_batch_plan_create: too many work items");
@@ -611,6 +613,14 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
 
   // Per-view tiles: frustum-major, 64 objects per tile.
   std::vector<std::vector<ViewTile>> per_view(n_frusta);
+  std::vector<uint64_t> view_words(n_frusta, 0);
+  uint64_t all_words = 0;
+  for (size_t k = 0; k < n_pairs; ++k) {
+    const uint64_t words = (groups[pairs[k].group].count + 63) / 64;
+    view_words[pairs[k].frustum] += words;
+    all_words += words;
+  }
+  for (uint32_t f = 0; f < n_frusta; ++f) per_view[f].reserve(view_words[f]);
   for (size_t k = 0; k < n_pairs; ++k) {
     const dpc_cull_pair& p = pairs[k];
     const dpc_group_range& g = groups[p.group];
@@ -627,6 +637,7 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
     }
   }
   std::vector<ViewTile> flat;
+  flat.reserve(all_words);
   plan->view_tile_begin.assign(n_frusta + 1, 0);
   for (uint32_t f = 0; f < n_frusta; ++f) {
     plan->view_tile_begin[f] = static_cast<uint32_t>(flat.size());
