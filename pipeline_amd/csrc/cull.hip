@@ -22,6 +22,7 @@ namespace {
 constexpr unsigned kCullThreads = 256;  // persistent streaming form
 constexpr unsigned kIndexedThreads = 512;  // plain form with an index array
 constexpr unsigned kPlainThreads = 1024;  // plain form without an index array
+constexpr unsigned kSmallThreads = 64;    // ... of short calls (launch_cull)
 
 // With Diff (the cull of Manager::cull, which the result diff follows), the
 // wave that stores mask word w also stores the number of bits in which it
@@ -45,8 +46,8 @@ __device__ __forceinline__ uint8_t changed_in_word(unsigned long long old_bits, 
 // shared by several objects, e.g. the leaves of a transform tree), plain cached
 // loads in 512-thread blocks measured fastest (19.3 us against 19.5-19.7 us with
 // 256 threads for the 2.37M objects of a 1M-node tree).
-template <bool Indexed, bool Diff>
-__global__ __launch_bounds__(Indexed ? kIndexedThreads : kPlainThreads) void cull_kernel(const float4* __restrict__ box_a,
+template <bool Indexed, bool Diff, unsigned Threads>
+__global__ __launch_bounds__(Threads) void cull_kernel(const float4* __restrict__ box_a,
                                                             const float2* __restrict__ box_b,
                                                             const uint32_t* __restrict__ xform, size_t n,
                                                             const float4* __restrict__ planes, size_t ld, Mat16 vp,
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(Indexed ? kIndexedThreads : kPlainThreads) void cul
                                                             const unsigned long long* __restrict__ old,
                                                             uint8_t* __restrict__ count)
 {
-  const size_t i = static_cast<size_t>(blockIdx.x) * (Indexed ? kIndexedThreads : kPlainThreads) + threadIdx.x;
+  const size_t i = static_cast<size_t>(blockIdx.x) * Threads + threadIdx.x;
   const bool writer = (threadIdx.x & (kWave - 1)) == 0 && i < n;  // lane 0 of a wave holding objects
   const unsigned long long old_bits = Diff && writer ? old[i >> 6] : 0ull;  // loaded with the objects
   const Slot s = make_slot(i, n, Indexed ? xform : nullptr, ld);
@@ -1014,15 +1015,29 @@ int launch_cull(const float* d_box_a, const float* d_box_b, const uint32_t* d_xf
     // calls lose by the waves they no longer have (700,000 with 4: 8.2 -> 8.4 us;
     // 400,000: 5.8 -> 6.3), and with a matrix to each object or two memory is the
     // bound (4,900,000: 72.8 -> 75.2 with one, 50.4 -> 50.8 with two).
-    if (d_xform && n_objects >= 1'400'000 && n_objects / 3 >= ld)
+    if (d_xform && n_objects >= 1'400'000 && n_objects / 3 >= ld) {
       hipLaunchKernelGGL((cull_pair_kernel<Diff>), dim3(grid_for((n_objects + 1) / 2, kPairThreads)), dim3(kPairThreads), 0,
                          s, a, b, d_xform, n_objects, p, ld, m, out, old, count);
-    else if (d_xform)
-      hipLaunchKernelGGL((cull_kernel<true, Diff>), dim3(grid_for(n_objects, kIndexedThreads)), dim3(kIndexedThreads), 0, s,
-                         a, b, d_xform, n_objects, p, ld, m, out, old, count);
+      return check_launch("cull_pair_kernel");
+    }
+    const auto launch = [&](auto kernel, unsigned threads) {
+      hipLaunchKernelGGL(kernel, dim3(grid_for(n_objects, threads)), dim3(threads), 0, s, a, b, d_xform, n_objects, p, ld, m,
+                         out, old, count);
+    };
+    // Without an index array, a workgroup of one wave in calls of up to 900,000
+    // objects: 10,000 objects in workgroups of 1024 threads occupy 10 CUs, sixteen
+    // waves each (the kernel: 10,000 objects 3.6 -> 2.8 us, 60,000 4.0 -> 3.2, 300,000
+    // 6.8 -> 5.6, 800,000 12.7 -> 12.1; two frames with their diffs over 300,000 21.4
+    // -> 19.3, 800,000 33.3 -> 31.4).  Longer calls wait for memory, and starting
+    // sixteen times as many workgroups costs more (1,048,576: 15.0 -> 15.7 us,
+    // 4,999,999: 65.3 -> 70.2).  With one, workgroups of 512 are spread well enough
+    // (two frames over 500,000, 4 to a matrix: 19.5 against 20.0).
+    if (d_xform)
+      launch(cull_kernel<true, Diff, kIndexedThreads>, kIndexedThreads);
+    else if (n_objects <= 900'000)
+      launch(cull_kernel<false, Diff, kSmallThreads>, kSmallThreads);
     else
-      hipLaunchKernelGGL((cull_kernel<false, Diff>), dim3(grid_for(n_objects, kPlainThreads)), dim3(kPlainThreads), 0,
-                         s, a, b, d_xform, n_objects, p, ld, m, out, old, count);
+      launch(cull_kernel<false, Diff, kPlainThreads>, kPlainThreads);
   } else {
     const size_t waves_per_block = kCullThreads / kWave;
     size_t blocks = static_cast<size_t>(device_cu_count()) * cfg.waves_per_cu / waves_per_block;

@@ -1,7 +1,8 @@
 """The single-view cull over a long array whose objects share matrices, where a wave
 takes two adjacent tiles: counts that end in the first or the second tile of a wave,
 on both sides of the lines where that form is taken, and indices outside the matrix
-array.  Masks, counts and changed indices against the oracle, bit for bit."""
+array.  Masks, counts and changed indices against the oracle, bit for bit.  And the
+line between workgroups of one wave and of many."""
 import numpy as np
 import pytest
 
@@ -49,3 +50,19 @@ def test_cull_pair_matches_oracle(n, share):
     index = np.flatnonzero(bits).astype(np.uint32)
     assert int(count.download()[0]) == index.size
     assert np.array_equal(changed.download()[:index.size], index)
+
+
+@pytest.mark.parametrize("share", [0, 4])
+@pytest.mark.parametrize("n", [1, 64, 65, 899_999, 900_000, 900_001])
+def test_cull_workgroup_sizes(n, share):
+    rng = np.random.default_rng(n + share)
+    k = max(n // share, 1) if share else n
+    lower, upper = scenes.random_boxes(rng, n, (-300.0, 300.0))
+    mats = scenes.trs_matrices(rng, k)
+    xform = np.minimum(np.arange(n) // share, k - 1).astype(np.uint32) if share else None
+    vp = scenes.perspective_vp((0, 0, 0), rng.normal(size=3), 60.0, 1.5, 0.1, 900.0)
+    got = dev.cull(dev.upload_scene(lower, upper, mats, xform), vp).download()
+    l4, e4 = scenes.extents(lower, upper)
+    want = orc.cull_obbs(orc.obb_build_group(l4, e4, np.arange(n) if xform is None else xform, mats), vp)
+    assert mismatches(got, want, n) == 0
+    assert n % 64 == 0 or int(got[-1]) >> (n % 64) == 0
