@@ -28,6 +28,7 @@
 // ahead of the item that is tested: without the 22 registers that takes, six
 // waves run per SIMD, and hide the loads themselves.
 #include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <numeric>
 #include <vector>
@@ -186,14 +187,31 @@ __device__ __forceinline__ uint32_t set_lane(uint32_t v, uint32_t to)
 // A run of kQuickRun frusta (at most) of a work item's list.
 template <int K>
 struct Run {
-  uint32_t todo, again;   // bit f: frustum f is to be tested; is to be tested once the queue is empty
+  uint32_t todo, again;   // bit f: frustum f is to be tested; is left for when the queue is empty
   uint32_t queued[K];     // bit f: word k of frustum f waits in the queue
   uint32_t lo[K], hi[K];  // lane 4 f: word k of frustum f
 };
 
+// Where the quick test decides little (boxes as large as what a view sees; object
+// matrices with a projective part, of which it decides nothing), the queue costs more
+// than testing every pair exactly: an undecided pair reads its object and its view
+// again, alone (500,003 objects x 32 frusta, nothing decided: 136 us, with every pair
+// tested exactly 66).  A full queue therefore ends a run: a frustum that leaves more
+// than kDenseLanes objects of 64 undecided goes to the exact test as a whole, with
+// those after it, where the words that wait were as dense (68 us; a third of the
+// matrices projective, 19 a word: 82 -> 68, and 112 with the line at 24 lanes; with it
+// at 8, boxes of which a word leaves 8 undecided: 41 -> 58).  The question is asked of a
+// full queue only: asked at every undecided word it cost the ordinary scene 8 %.
+constexpr uint32_t kDenseLanes = 16;
+constexpr uint32_t kExact = 1u << 31;
+// After an item of whose list less than a quarter was done before that, a wave takes
+// this many items through the exact test without trying the quick one (68.4 us; with
+// every item tried 70.7, with one in eight 68.4).
+constexpr uint32_t kExactItems = 3;
+
 // Tests the wave's objects against frustum F of a run.  A word with undecided
 // objects goes to the queue; without room for them the frustum and those after it
-// are left for `again`.
+// are left (kExact: to the exact test).
 template <int F, int K>
 __device__ __forceinline__ void test_frustum(Run<K>& run, const WorkItem& item, const TileObjects<K>& t,
                                              const QuickRows& rows, const KPair& pair, uint32_t lane, Queue<K>& queue,
@@ -216,6 +234,7 @@ __device__ __forceinline__ void test_frustum(Run<K>& run, const WorkItem& item, 
   for (int k = 0; k < K; ++k) n_open += static_cast<uint32_t>(__builtin_popcountll(open[k]));
   if (waiting + n_open > Queue<K>::kCapacity) {
     run.again = run.todo & (~0u << F);
+    if (n_open > kDenseLanes * K && waiting > kDenseLanes * words) run.again |= kExact;
     run.todo = 0;
     return;
   }
@@ -225,7 +244,7 @@ __device__ __forceinline__ void test_frustum(Run<K>& run, const WorkItem& item, 
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     if (open[k] == 0) continue;
-    if ((open[k] >> lane) & 1) {
+    if (__builtin_amdgcn_inverse_ballot_w64(open[k])) {
       const uint64_t object = item.first_object + lane + kWave * k;
       const uint32_t at = waiting + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(open[k] >> 32),
                                                               __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(open[k]), 0u));
@@ -256,17 +275,19 @@ __device__ __forceinline__ void test_run(Run<K>& run, const WorkItem& item, cons
 // frustum and 64 objects.  Words that the quick test (quick_cull.hpp) decides whole
 // are stored together, a run's in one instruction; the others wait in the queue.
 // pair: the first run's entries of the item's list.  view_of(p0, p, frustum) gives
-// the lane the QuickView of the item's p-th frustum, in the run from p0 on; with
-// `last` the queue is drained before the return.
+// the lane the QuickView of the item's p-th frustum, in the run from p0 on.  Returns
+// how many of the list's frusta are done: where not all are, the next ones are left to
+// test_exact.
 template <int K, class ViewOf>
-__device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObjects<K>& t, KPair pair, uint32_t lane,
-                                            const KPair* __restrict__ pairs, const SceneDev* __restrict__ scenes,
-                                            const float* __restrict__ vps, unsigned long long* __restrict__ masks,
-                                            Queue<K>& queue, uint32_t& waiting, uint32_t& words, bool last,
-                                            ViewOf&& view_of)
+__device__ __forceinline__ uint32_t test_frusta(const WorkItem& item, const TileObjects<K>& t, KPair pair, uint32_t lane,
+                                                const KPair* __restrict__ pairs, const SceneDev* __restrict__ scenes,
+                                                const float* __restrict__ vps, unsigned long long* __restrict__ masks,
+                                                Queue<K>& queue, uint32_t& waiting, uint32_t& words, ViewOf&& view_of)
 {
-  for (uint32_t p0 = 0;;) {
-    const uint32_t left = item.pair_count - p0, n = left < kQuickRun ? left : kQuickRun;
+  uint32_t p0 = 0;
+  for (;;) {
+    const uint32_t left = item.pair_count - p0;
+    uint32_t n = left < kQuickRun ? left : kQuickRun;
     const QuickRows rows = quick_rows(view_of(p0, p0 + min(lane / 4 % kQuickRun, n - 1), pair.frustum), lane % 4);
     const KPair next = load_pairs(pairs, item, p0 + kQuickRun, lane);
     Run<K> run = {};
@@ -274,6 +295,10 @@ __device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObje
     for (;;) {
       test_run<0, K>(run, item, t, rows, pair, lane, queue, waiting, words);
       if (run.again == 0) break;
+      if (run.again & kExact) {
+        n = static_cast<uint32_t>(__builtin_ctz(run.again));
+        break;
+      }
       drain<K>(queue, waiting, words, lane, scenes, vps, masks);
       waiting = words = 0;
       run.todo = run.again;
@@ -286,13 +311,38 @@ __device__ __forceinline__ void test_frusta(const WorkItem& item, const TileObje
       if (lane % 4 == 0 && lane / 4 < n && !((run.queued[k] >> (lane / 4)) & 1))
         masks[pair.mask_word + item.tile_word + k] = static_cast<unsigned long long>(run.hi[k]) << 32 | run.lo[k];
     }
-    if (left <= kQuickRun) break;
-    p0 += kQuickRun;
+    p0 += n;
+    if (p0 >= item.pair_count || n < kQuickRun) break;
     pair = next;
   }
-  if (last) {
-    drain<K>(queue, waiting, words, lane, scenes, vps, masks);
-    waiting = words = 0;
+  return p0;
+}
+
+// The exact test of a work item's objects against the frusta [first, end) of its list,
+// each in scalar registers.  The objects are read again: kept across the quick test they
+// would take the registers of a wave per SIMD.
+template <int K>
+__device__ __forceinline__ void test_exact(WorkItem item, uint32_t first, uint32_t end, uint32_t lane,
+                                           const KPair* __restrict__ pairs, const SceneDev* __restrict__ scenes,
+                                           const float* __restrict__ vps, unsigned long long* __restrict__ masks)
+{
+  // (as new values: the scene and addresses of the first read would otherwise be kept)
+  asm volatile("" : "+s"(item.scene), "+s"(item.first_object), "+v"(lane));
+  Slot slot[K];
+  RawObj raw[K];
+  load_objects<K>(scenes, item, lane, slot, raw);
+  Obb o[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) o[k] = obb_of(raw[k]);
+  for (uint32_t p = first; p < end; ++p) {
+    const KPair pair = pairs[item.pair_begin + p];
+    Mat16 m;
+    load_vp(vps, pair.frustum, m);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const unsigned long long bits = ballot(slot_visible(slot[k], obb_visible(o[k], m.m)));
+      if (k == 0 || static_cast<uint32_t>(kWave * k) < item.count) masks[pair.mask_word + item.tile_word + k] = bits;
+    }
   }
 }
 
@@ -334,37 +384,47 @@ __global__ __launch_bounds__(256, K == 1 ? (Table ? 6 : 5) : K == 2 ? 4 : 2) voi
   const uint32_t n_waves = gridDim.x * waves_per_block;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   uint32_t it = blockIdx.x * waves_per_block + wave;
-  uint32_t waiting = 0, words = 0;
+  uint32_t waiting = 0, words = 0, exact = 0;
   for (bool first = true;; first = false) {
     const WorkItem item = items[it < n_items ? it : 0];  // (n_items >= 1)
-    Slot slot[K];
-    RawObj raw[K];
-    load_objects<K>(scenes, item, lane, slot, raw);
-    const KPair pair = load_pairs(pairs, item, 0, lane);
-    if (first) {  // the table is built while the first objects are in flight
-      if (Table) {
-        for (uint32_t f = threadIdx.x; f < n_frusta; f += blockDim.x) {
-          Mat16 m;
-          load_vp(vps, f, m);
-          table[f] = quick_view(m.m);
+    uint32_t done = 0;
+    if (__builtin_expect(exact != 0, 0)) {
+      --exact;
+    } else {
+      Slot slot[K];
+      RawObj raw[K];
+      load_objects<K>(scenes, item, lane, slot, raw);
+      const KPair pair = load_pairs(pairs, item, 0, lane);
+      if (first) {  // the table is built while the first objects are in flight
+        if (Table) {
+          uint32_t f = threadIdx.x;
+          asm volatile("" : "+v"(f));  // (the comparison stays here, not in registers of the whole loop)
+          for (; f < n_frusta; f += blockDim.x) {
+            Mat16 m;
+            load_vp(vps, f, m);
+            table[f] = quick_view(m.m);
+          }
+          lds_barrier();
         }
-        lds_barrier();
+        if (it >= n_items) return;  // (a wave without an item helped with the table)
       }
-      if (it >= n_items) return;  // (a wave without an item helped with the table)
+      TileObjects<K> objects;
+      quick_objects<K>(slot, raw, objects);
+      auto view_of = [&](uint32_t p0, uint32_t p, uint32_t f) -> const QuickView& {
+        if (Table) return table[f];
+        if (p0 % kWave == 0)
+          list_views(pairs + item.pair_begin + p0, item.pair_count - p0, vps, lane, &table[wave * kWave]);
+        return table[wave * kWave + p % kWave];
+      };
+      done = test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, view_of);
+      if (done * 4 < item.pair_count) exact = kExactItems;
     }
-    TileObjects<K> objects;
-    quick_objects<K>(slot, raw, objects);
-    const bool last = it + n_waves >= n_items;
-    auto view_of = [&](uint32_t p0, uint32_t p, uint32_t f) -> const QuickView& {
-      if (Table) return table[f];
-      if (p0 % kWave == 0)
-        list_views(pairs + item.pair_begin + p0, item.pair_count - p0, vps, lane, &table[wave * kWave]);
-      return table[wave * kWave + p % kWave];
-    };
-    test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, last, view_of);
-    if (last) break;
+    if (__builtin_expect(done < item.pair_count, 0))
+      test_exact<K>(item, done, item.pair_count, lane, pairs, scenes, vps, masks);
     it += n_waves;
+    if (it >= n_items) break;
   }
+  drain<K>(queues[wave], waiting, words, lane, scenes, vps, masks);
 }
 
 // ---- serving form -----------------------------------------------------------
@@ -380,19 +440,41 @@ __global__ __launch_bounds__(256, K == 1 ? (Table ? 6 : 5) : K == 2 ? 4 : 2) voi
 constexpr uint32_t kServeViews = 64;  // frusta of a request, at most (dpc_server_submit)
 static_assert(kServeViews <= kWave, "one lane per frustum");
 
+// A wave's current entry: its fields in the lanes of one register, each read where it
+// is used (as scalars beside the loop's state they spill: 4 scenes of 500,003 objects,
+// 32 views each, 282 -> 291 us a tick).
+struct EntryLanes {
+  uint32_t v;  // lane l: word l % 8 of the ServeEntry
+  __device__ __forceinline__ uint32_t get(size_t offset) const
+  {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(offset / 4)));
+  }
+  __device__ __forceinline__ uint32_t pair_begin() const { return get(offsetof(ServeEntry, pair_begin)); }
+  __device__ __forceinline__ uint32_t pair_count() const { return get(offsetof(ServeEntry, pair_count)); }
+  __device__ __forceinline__ uint32_t tiles() const { return get(offsetof(ServeEntry, tiles)); }
+};
+static_assert(sizeof(ServeEntry) == 32, "eight words");
+
+__device__ __forceinline__ EntryLanes entry_lanes(const ServeEntry* __restrict__ entries, uint32_t a, uint32_t lane)
+{
+  return {reinterpret_cast<const uint32_t*>(&entries[a])[lane % 8]};
+}
+
 // The part of an entry's tile that a wave tests: `count` frusta from the entry's
 // frustum `first` on.
 template <int K>
-__device__ __forceinline__ WorkItem serve_item(const ServeEntry& e, uint32_t tile, uint32_t first, uint32_t count)
+__device__ __forceinline__ WorkItem serve_item(const EntryLanes& e, uint32_t tile, uint32_t first, uint32_t count)
 {
   WorkItem w;
   w.first_object = static_cast<uint64_t>(tile) * (kWave * K);
-  const uint64_t left = e.objects - w.first_object;
+  const uint64_t objects = static_cast<uint64_t>(e.get(offsetof(ServeEntry, objects) + 4)) << 32 |
+                           e.get(offsetof(ServeEntry, objects));
+  const uint64_t left = objects - w.first_object;
   w.count = static_cast<uint32_t>(left < static_cast<uint64_t>(kWave * K) ? left : static_cast<uint64_t>(kWave * K));
   w.tile_word = tile * K;
-  w.pair_begin = e.pair_begin + first;
+  w.pair_begin = e.pair_begin() + first;
   w.pair_count = count;
-  w.scene = e.scene;
+  w.scene = e.get(offsetof(ServeEntry, scene));
   w.pad = 0;
   return w;
 }
@@ -420,32 +502,49 @@ __global__ __launch_bounds__(256, 4) void cull_serve_kernel(const ServeEntry* __
     a += __popcll(ballot(entries[k < n_entries ? k : 0].cost_begin <= c0 && k < n_entries));
   }
   a = __builtin_amdgcn_readfirstlane(a - 1);
-  ServeEntry e = entries[a];
   uint32_t left = static_cast<uint32_t>(c1 - c0);  // (at most a few tiles' frusta: c1 - c0 is total_cost / W)
-  uint32_t tile = static_cast<uint32_t>((c0 - e.cost_begin) / e.pair_count);
-  uint32_t first = static_cast<uint32_t>((c0 - e.cost_begin) % e.pair_count);
-  uint32_t waiting = 0, words = 0, viewed = ~0u;
+  uint32_t tile = static_cast<uint32_t>((c0 - entries[a].cost_begin) / entries[a].pair_count);
+  uint32_t first = static_cast<uint32_t>((c0 - entries[a].cost_begin) % entries[a].pair_count);
+  EntryLanes e = entry_lanes(entries, a, lane);
+  bool viewed = false;
+  uint32_t waiting = 0, words = 0, exact = 0;
   for (;;) {
-    const uint32_t rest = e.pair_count - first, count = rest < left ? rest : left;
+    const uint32_t rest = e.pair_count() - first, count = rest < left ? rest : left;
     const WorkItem item = serve_item<K>(e, tile, first, count);
-    Slot slot[K];
-    RawObj raw[K];
-    load_objects<K>(scenes, item, lane, slot, raw);
-    const KPair pair = load_pairs(pairs, item, 0, lane);
-    if (viewed != a) {  // the entry's QuickViews, one per lane, while its first objects are in flight
-      list_views(pairs + e.pair_begin, e.pair_count, vps, lane, views[block_wave]);
-      viewed = a;
+    uint32_t done = 0, end = count;
+    if (__builtin_expect(exact != 0, 0)) {
+      --exact;
+    } else {
+      Slot slot[K];
+      RawObj raw[K];
+      load_objects<K>(scenes, item, lane, slot, raw);
+      const KPair pair = load_pairs(pairs, item, 0, lane);
+      if (!viewed) {  // the entry's QuickViews, one per lane, while its first objects are in flight
+        list_views(pairs + e.pair_begin(), e.pair_count(), vps, lane, views[block_wave]);
+        viewed = true;
+      }
+      TileObjects<K> objects;
+      quick_objects<K>(slot, raw, objects);
+      const QuickView* const list = &views[block_wave][first];
+      done = test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[block_wave], waiting, words,
+                            [&](uint32_t, uint32_t p, uint32_t) -> const QuickView& { return list[p]; });
+      // (what is left, to the end of the run: what the list's later views see may be decided again)
+      end = min(done / kQuickRun * kQuickRun + kQuickRun, count);
+      if (done * 4 < end) exact = kExactItems;
     }
-    TileObjects<K> objects;
-    quick_objects<K>(slot, raw, objects);
-    left -= count;
-    const QuickView* const list = &views[block_wave][first];
-    test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[block_wave], waiting, words, left == 0,
-                   [&](uint32_t, uint32_t p, uint32_t) -> const QuickView& { return list[p]; });
+    if (__builtin_expect(done < end, 0)) test_exact<K>(item, done, end, lane, pairs, scenes, vps, masks);
+    left -= end;
     if (left == 0) break;
+    first += end;
+    asm volatile("" : "+v"(e.v));  // (as a new value: what was read of it would otherwise be kept)
+    if (first < e.pair_count()) continue;
     first = 0;
-    for (++tile; tile >= e.tiles; tile = 0) e = entries[++a];  // (pairs are left: an entry with tiles follows)
+    for (++tile; tile >= e.tiles(); tile = 0) {  // (pairs are left: an entry with tiles follows)
+      e = entry_lanes(entries, ++a, lane);
+      viewed = false;
+    }
   }
+  drain<K>(queues[block_wave], waiting, words, lane, scenes, vps, masks);
 }
 
 // Plain per-view launch: one wave per 64-object tile, the frustum by value.
