@@ -46,9 +46,21 @@
 // The bounds take 80 u T for z + w and w - z and 160 u T for x and y, and the tests
 // for `visible` 80 and twice that: 2^-17 s3 and 2^-17 sw (128 u) times 0.625 and 1.25
 // of n3 and n4.  The 2^-90 and 2^-117 added to the object's factors cover underflow.
-// Operands of 2^56 (matrix) or 2^60 (object) and above, matrices whose rows 0-2 lie
-// below 2^-47, infinities and NaN make eps infinite or NaN, and every comparison
-// below false: undecided.  So does an object whose edges have a w component.
+//
+// What the bound does not cover is left undecided: operands of 2^56 (matrix) or 2^60
+// (object) and above, infinities and NaN, matrices whose rows 0-2 lie below 2^-47, and
+// objects whose edges have a w component make n3, n4 or s3 infinite, and every bound
+// +infinity or NaN.  No comparison for `culled` holds with one.  The test for `visible`
+// takes its operands from medians, which drop a NaN (quick_med3):
+//   both bounds of z infinite   eps is +infinity, below neither of z + w and w - z
+//   one NaN (eps -infinity)     it comes from the radius, a norm or sw times n4.
+//     The radius is NaN only where an edge has an infinite or NaN component (finite
+//     ones overflow to magnitudes): that component of the centre is too, every
+//     output is infinite or NaN, and `far` +infinity, below nothing.
+//     A norm is NaN only where the column of its own output, z + w or w - z, has a
+//     NaN; sw times n4 only where p.w is NaN, or infinite over a row 3 of zeros.  The
+//     output is then NaN and `near` -infinity, above nothing.
+//   x or y NaN (dropped by `far`)  only with operands that make both bounds so.
 #pragma once
 
 #include <cstdint>
@@ -122,6 +134,18 @@ DPC_HD QuickObj quick_obj(const V4& p, const V4& ex, const V4& ey, const V4& ez)
   return q;
 }
 
+// v_med3_f32, in one instruction where a maximum first quiets its operands: the median,
+// and with a NaN among them the smallest of the others.
+DPC_HD float quick_med3(float a, float b, float c)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_fmed3f(a, b, c);
+#else
+  if (a != a || b != b || c != c) return __builtin_fminf(__builtin_fminf(a, b), c);
+  return __builtin_fmaxf(__builtin_fminf(a, b), __builtin_fminf(__builtin_fmaxf(a, b), c));
+#endif
+}
+
 // The largest magnitude of the elements of row 3, or of rows 0-2, as a float:
 // magnitudes compare as their bits do, NaN above infinity (integer operations,
 // which run on the scalar unit for a wave-uniform matrix).
@@ -180,16 +204,11 @@ template <class M, class Less>
 DPC_HD QuickResult<M> quick_decide(const float (&out)[4], const float (&bound)[4], Less&& less)
 {
   const float ax = __builtin_fabsf(out[0]), ay = __builtin_fabsf(out[1]), l = out[2], h = out[3];
-#ifdef __HIP_DEVICE_COMPILE__
-  // (the median with an infinity that the compiler does not see: one instruction,
-  // where a maximum first quiets its operands)
   float inf = __builtin_inff();
-  asm("" : "+s"(inf));
-  const float far = __builtin_amdgcn_fmed3f(ax, ay, inf), near = __builtin_amdgcn_fmed3f(l, h, -inf);
-  const float eps = __builtin_amdgcn_fmed3f(bound[2], bound[3], -inf);
-#else
-  const float far = ax < ay ? ay : ax, near = l < h ? l : h, eps = bound[2] < bound[3] ? bound[2] : bound[3];
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+s"(inf));  // (the compiler would take the medians for a maximum and minima)
 #endif
+  const float far = quick_med3(ax, ay, inf), near = quick_med3(l, h, -inf), eps = quick_med3(bound[2], bound[3], -inf);
   const float w = l + h, aw = __builtin_fabsf(w);
   QuickResult<M> r;
   r.visible = less(far, quick_fma(-2.0f, eps, w)) & less(eps, near);
