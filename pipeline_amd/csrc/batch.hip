@@ -479,6 +479,20 @@ __device__ __forceinline__ WorkItem serve_item(const EntryLanes& e, uint32_t til
   return w;
 }
 
+// The kernel's LDS, and the workgroups of it that a CU holds: its 160 KB are given out
+// in units of 1280 bytes, so of 32 KB four fit, not five (hipOccupancyMaxActiveBlocks-
+// PerMultiprocessor says five; a fifth takes as long as of 33,280 bytes).
+template <int K>
+struct ServeLds {
+  Queue<K> queues[kBatchWaves];
+  QuickView views[kBatchWaves][kServeViews];  // of each wave's current entry
+};
+constexpr uint32_t lds_blocks(size_t bytes) { return static_cast<uint32_t>(160 * 1024 / ((bytes + 1279) / 1280 * 1280)); }
+static_assert(lds_blocks(32000) == 5 && lds_blocks(32768) == 4, "units of 1280 bytes");
+template <int K>
+constexpr uint32_t kServeBlocks = lds_blocks(sizeof(ServeLds<K>));
+static_assert(kServeBlocks<1> == 4 && kServeBlocks<2> == 4, "launch_serve's times are of four");
+
 template <int K>
 __global__ __launch_bounds__(256, 4) void cull_serve_kernel(const ServeEntry* __restrict__ entries, uint32_t n_entries,
                                                          uint64_t total_cost, const KPair* __restrict__ pairs,
@@ -486,8 +500,9 @@ __global__ __launch_bounds__(256, 4) void cull_serve_kernel(const ServeEntry* __
                                                          const float* __restrict__ vps,
                                                          unsigned long long* __restrict__ masks)
 {
-  __shared__ Queue<K> queues[kBatchWaves];
-  __shared__ QuickView views[kBatchWaves][kServeViews];  // of the wave's current entry
+  __shared__ ServeLds<K> lds;
+  auto& queues = lds.queues;
+  auto& views = lds.views;
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t waves_per_block = blockDim.x / kWave;
   const uint64_t W = static_cast<uint64_t>(gridDim.x) * waves_per_block;
@@ -928,9 +943,12 @@ int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost,
   const uint32_t waves_per_block = 4;
   // A small batch is split into runs of a length that gives about five waves per CU,
   // as a batch plan's lists are (dpc_batch_plan_create); a large one into as many
-  // runs as the device holds waves (LDS: five workgroups per CU).
+  // runs as the device holds waves: with a workgroup per CU more, a fifth of the equal
+  // runs starts when the others end (1,000,003 objects x 32 views of which the quick
+  // test decides nothing: 307 us a tick, 282 without; ordinary 168 to 175, 168).
   const uint64_t cus = device_cu_count();
-  uint64_t waves = cus * (waves_per_cu ? waves_per_cu : 20);
+  const uint32_t held = waves_per_block * (objects_per_lane == 2 ? kServeBlocks<2> : kServeBlocks<1>);
+  uint64_t waves = cus * (waves_per_cu ? waves_per_cu : held);
   waves = std::min(waves, total_cost / std::clamp<uint64_t>((total_cost + 5 * cus - 1) / (5 * cus), 2, 16));
   if (waves == 0) waves = 1;
   const uint64_t blocks = (waves + waves_per_block - 1) / waves_per_block;
