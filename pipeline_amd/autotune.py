@@ -20,6 +20,7 @@ import ctypes as C
 import itertools
 import json
 import math
+import re
 import sys
 import time
 from pathlib import Path
@@ -56,13 +57,16 @@ def load_table(arch: str | None = None) -> dict:
 
 
 def best_batch_config(objects: int, tests: int, frusta: int, arch: str | None = None):
-    t = load_table(arch).get("batch", {})
-    entry = t.get(batch_bucket(objects, tests, frusta))
-    if entry is None and t:
-        # nearest bucket by test count
-        key = min(t, key=lambda k: abs(int(k.split("tests2^")[1].split("-")[0]) - _bucket(tests)))
-        entry = t[key]
-    return _lib.BatchConfig(*entry["config"]) if entry else None
+    """The tuned config of the nearest measured shape, or None (the plan's defaults)
+    where none lies within a factor of about two in objects, tests and frusta: what
+    is best for 2 M objects is slow for 20 k, whose lists the plan cuts shorter."""
+    near = []
+    for key, entry in load_table(arch).get("batch", {}).items():
+        o, t, f = map(int, re.fullmatch(r"obj2\^(\d+)-tests2\^(\d+)-frusta(\d+)", key).groups())
+        off = (abs(o - _bucket(objects)), abs(t - _bucket(tests)), abs(math.log2(max(f, 1) / max(frusta, 1))))
+        if max(off) <= 1:
+            near.append((sum(off), key, entry))
+    return _lib.BatchConfig(*min(near, key=lambda n: n[:2])[2]["config"]) if near else None
 
 
 def best_cull_config(objects: int, arch: str | None = None):
