@@ -179,12 +179,13 @@ typedef struct dpc_batch_config {
   uint32_t objects_per_lane; /* 1, 2 or 4: a wave owns 64*objects_per_lane objects */
   uint32_t block_threads;    /* 64, 128, 256 */
   uint32_t waves_per_cu;     /* persistent grid size = CUs * waves_per_cu / waves per block */
-  uint32_t max_frusta_per_item; /* split a tile's frustum list into chunks of this size (0 = the plan chooses) */
+  uint32_t max_frusta_per_item; /* split a tile's frustum list into chunks of this size (0 = no split) */
 } dpc_batch_config;
 
 typedef struct dpc_batch_plan dpc_batch_plan;
 
-/* Builds the work list (tiles sorted by cost) and uploads it.  cfg NULL = defaults. */
+/* Builds the work list (tiles sorted by cost) and uploads it.  cfg NULL = defaults,
+ * with chunks of a size that the plan chooses by the amount of work. */
 int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const dpc_cull_pair* pairs,
                           size_t n_pairs, uint32_t n_frusta, const dpc_batch_config* cfg, dpc_batch_plan** plan);
 int dpc_batch_plan_destroy(dpc_batch_plan* plan);

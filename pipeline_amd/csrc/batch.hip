@@ -672,7 +672,7 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   for (size_t g = 0; g < n_groups; ++g) group_pair_begin[g + 1] += group_pair_begin[g];
 
   const uint64_t tile_objects = static_cast<uint64_t>(kWave) * c.objects_per_lane;
-  if (c.max_frusta_per_item == 0) {
+  if (!cfg) {
     // Where the tiles alone would leave the device idle, lists are split into
     // slices of a length that gives about five work items per CU, of two views at
     // least (79 tiles x 64 views: 10.3 us in slices of 32, 6.0 of 4, 6.3 of 2; 625 x
@@ -695,7 +695,8 @@ int dpc_batch_plan_create(const dpc_group_range* groups, size_t n_groups, const 
   for (size_t g = 0; g < n_groups; ++g) {
     const uint64_t pb = group_pair_begin[g], pe = group_pair_begin[g + 1];
     if (pb == pe || groups[g].count == 0) continue;
-    const uint64_t slices = (pe - pb + c.max_frusta_per_item - 1) / c.max_frusta_per_item;
+    const uint64_t most = c.max_frusta_per_item ? c.max_frusta_per_item : pe - pb;
+    const uint64_t slices = (pe - pb + most - 1) / most;
     const uint64_t chunk = (pe - pb + slices - 1) / slices;
     for (uint64_t t0 = 0; t0 < groups[g].count; t0 += tile_objects) {
       const uint32_t cnt = static_cast<uint32_t>(std::min<uint64_t>(tile_objects, groups[g].count - t0));
