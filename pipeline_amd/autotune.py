@@ -153,9 +153,20 @@ def batch_candidates(quick=False):
     ks = (1, 2) if quick else (1, 2, 4)
     blocks = (256,) if quick else (64, 128, 256)
     waves = (8, 16, 24) if quick else (4, 8, 12, 16, 24, 32)
-    chunks = (0, 4) if quick else (0, 2, 4, 8)
+    chunks = (0, 16) if quick else (0, 2, 4, 8, 16, 64)
     for k, b, w, c in itertools.product(ks, blocks, waves, chunks):
         yield (k, b, w, c)
+
+
+DEFAULT_SHAPE = [1, 256, 24]  # of a plan without a config
+
+
+def _best(rows):
+    """The fastest row; the default shape where it comes within 2 %, about what two
+    runs of a candidate differ by."""
+    fastest = min(rows, key=lambda r: r["us"])
+    default = min((r for r in rows if r["config"][:3] == DEFAULT_SHAPE), key=lambda r: r["us"], default=None)
+    return default if default and default["us"] <= 1.02 * fastest["us"] else fastest
 
 
 def tune_batch(bs: scenes.BatchedScene, candidates=None, log=print):
@@ -189,9 +200,7 @@ def tune_batch(bs: scenes.BatchedScene, candidates=None, log=print):
     d_vps.free()
     masks.free()
     stream.destroy()
-    good = [r for r in rows if r["ok"]]
-    best = min(good, key=lambda r: r["us"])
-    return best, rows
+    return _best([r for r in rows if r["ok"]]), rows
 
 
 def main(argv=None):

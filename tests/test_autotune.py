@@ -21,3 +21,16 @@ def test_only_near_shapes_are_tuned(table, objects, tests, frusta, want):
 
 def test_no_table():
     assert autotune.best_batch_config(1 << 21, 1 << 23, 64, "an arch without a table") is None
+
+
+def test_candidates_hold_whole_lists_and_the_plans_own_chunk():
+    for quick in (False, True):
+        chunks = {c[3] for c in autotune.batch_candidates(quick)}
+        assert {0, 16} <= chunks
+    assert 64 in {c[3] for c in autotune.batch_candidates()}
+
+
+@pytest.mark.parametrize("default_us,want", [(36.5, [1, 256, 24, 16]), (37.0, [2, 256, 16, 0])])
+def test_default_shape_wins_within_two_percent(default_us, want):
+    rows = [{"config": c, "us": us} for c, us in (([2, 256, 16, 0], 36.0), ([1, 256, 24, 4], 50.0), ([1, 256, 24, 16], default_us))]
+    assert autotune._best(rows)["config"] == want
