@@ -384,43 +384,46 @@ __global__ __launch_bounds__(256, K == 1 ? (Table ? 6 : 5) : K == 2 ? 4 : 2) voi
   const uint32_t n_waves = gridDim.x * waves_per_block;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   uint32_t it = blockIdx.x * waves_per_block + wave;
-  uint32_t waiting = 0, words = 0, exact = 0;
+  uint32_t waiting = 0, words = 0;
   for (bool first = true;; first = false) {
-    const WorkItem item = items[it < n_items ? it : 0];  // (n_items >= 1)
-    uint32_t done = 0;
-    if (__builtin_expect(exact != 0, 0)) {
-      --exact;
-    } else {
-      Slot slot[K];
-      RawObj raw[K];
-      load_objects<K>(scenes, item, lane, slot, raw);
-      const KPair pair = load_pairs(pairs, item, 0, lane);
-      if (first) {  // the table is built while the first objects are in flight
-        if (Table) {
-          uint32_t f = threadIdx.x;
-          asm volatile("" : "+v"(f));  // (the comparison stays here, not in registers of the whole loop)
-          for (; f < n_frusta; f += blockDim.x) {
-            Mat16 m;
-            load_vp(vps, f, m);
-            table[f] = quick_view(m.m);
-          }
-          lds_barrier();
+    WorkItem item = items[it < n_items ? it : 0];  // (n_items >= 1)
+    Slot slot[K];
+    RawObj raw[K];
+    load_objects<K>(scenes, item, lane, slot, raw);
+    const KPair pair = load_pairs(pairs, item, 0, lane);
+    if (first) {  // the table is built while the first objects are in flight
+      if (Table) {
+        uint32_t f = threadIdx.x;
+        asm volatile("" : "+v"(f));  // (the comparison stays here, not in registers of the whole loop)
+        for (; f < n_frusta; f += blockDim.x) {
+          Mat16 m;
+          load_vp(vps, f, m);
+          table[f] = quick_view(m.m);
         }
-        if (it >= n_items) return;  // (a wave without an item helped with the table)
+        lds_barrier();
       }
-      TileObjects<K> objects;
-      quick_objects<K>(slot, raw, objects);
-      auto view_of = [&](uint32_t p0, uint32_t p, uint32_t f) -> const QuickView& {
-        if (Table) return table[f];
-        if (p0 % kWave == 0)
-          list_views(pairs + item.pair_begin + p0, item.pair_count - p0, vps, lane, &table[wave * kWave]);
-        return table[wave * kWave + p % kWave];
-      };
-      done = test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, view_of);
-      if (done * 4 < item.pair_count) exact = kExactItems;
+      if (it >= n_items) return;  // (a wave without an item helped with the table)
     }
-    if (__builtin_expect(done < item.pair_count, 0))
-      test_exact<K>(item, done, item.pair_count, lane, pairs, scenes, vps, masks);
+    TileObjects<K> objects;
+    quick_objects<K>(slot, raw, objects);
+    auto view_of = [&](uint32_t p0, uint32_t p, uint32_t f) -> const QuickView& {
+      if (Table) return table[f];
+      if (p0 % kWave == 0)
+        list_views(pairs + item.pair_begin + p0, item.pair_count - p0, vps, lane, &table[wave * kWave]);
+      return table[wave * kWave + p % kWave];
+    };
+    uint32_t done =
+        test_frusta<K>(item, objects, pair, lane, pairs, scenes, vps, masks, queues[wave], waiting, words, view_of);
+    if (__builtin_expect(done < item.pair_count, 0)) {
+      // (the next items here too: asked for at each item, they cost a short launch 0.1 us)
+      for (uint32_t more = done * 4 < item.pair_count ? kExactItems : 0;; --more) {
+        test_exact<K>(item, done, item.pair_count, lane, pairs, scenes, vps, masks);
+        if (more == 0 || it + n_waves >= n_items) break;
+        it += n_waves;
+        item = items[it];
+        done = 0;
+      }
+    }
     it += n_waves;
     if (it >= n_items) break;
   }
