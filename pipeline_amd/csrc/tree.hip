@@ -655,14 +655,6 @@ struct dpc_tree_plan {
 
 namespace {
 
-// Threads of a tile workgroup where the caller leaves them to the plan.  Smaller
-// workgroups split a tree over more CUs, shorten each tile's steps and mix the
-// reads of one tile with the writes of another; larger ones recompute fewer
-// shared ancestors.  Full propagation with 256 / 512 / 1024 threads: 10,000 nodes
-// 5.9 / 5.9 / 6.2 us, 50,000 7.1 / 7.1 / 7.2, 100,000 8.7 / 8.2 / 8.2, 250,007
-// 12.7 / 11.7 / 11.9, 500,000 15.8 / 15.1 / 15.8, 700,000 25.0 / 24.6 / 29.6 (1 %
-// dirty 18.6 / 19.5 / 26.0), 1,000,000 34.4 / 35.8 / 36.1.
-uint32_t default_tile_threads(uint64_t slots) { return slots > 75000 && slots < 600000 ? 512 : 256; }
 constexpr size_t kMaxRunPasses = 32;
 
 template <bool HasDirty>
@@ -782,18 +774,20 @@ int dpc_tree_plan_create(const uint32_t* h_parent_slot, size_t ld, const uint64_
     return set_error(DPC_ERR_INVALID_ARGUMENT, "dpc_tree_plan_create: levels end beyond ld");
   if (tile_slots != 0 && tile_slots != 256 && tile_slots != 512 && tile_slots != 1024)
     return set_error(DPC_ERR_INVALID_ARGUMENT, "dpc_tree_plan_create: tile_slots must be 0, 256, 512 or 1024");
+  const tileplan::Shape shape =
+      tile_slots ? tileplan::Shape{tile_slots, 4} : tileplan::default_shape(h_level_offsets[n_levels]);
   if (n_levels == 0) {
     // a tree that holds only its root: propagation has nothing to compute
     // (Tree::compute visits no level and notifies an empty change set)
     auto plan = std::make_unique<dpc_tree_plan>();
     plan->ld = ld;
-    plan->threads = tile_slots ? tile_slots : default_tile_threads(h_level_offsets[n_levels]);
+    plan->threads = shape.threads;
     *out = plan.release();
     return DPC_OK;
   }
   auto plan = std::make_unique<dpc_tree_plan>();
   plan->ld = ld;
-  plan->threads = tile_slots ? tile_slots : default_tile_threads(h_level_offsets[n_levels]);
+  plan->threads = shape.threads;
   const uint32_t max_ring = tile_max_ring(plan->threads);
   // workgroups the device holds at once: CUs x tile workgroups per CU
   int dev = 0, cus = 0, per_cu = 0;
@@ -823,7 +817,7 @@ int dpc_tree_plan_create(const uint32_t* h_parent_slot, size_t ld, const uint64_
   const size_t run_passes = ld <= kMaxBufferSlots ? kMaxRunPasses : 1;
   const std::vector<tileplan::Step> sched =
       tileplan::schedule(h_parent_slot, h_level_offsets, n_levels, plan->threads, max_ring, capacity, kLdsNodes,
-                         kMaxLevelsPerSmall, run_passes);
+                         kMaxLevelsPerSmall, run_passes, 64, shape.last_steps);
   for (const auto& ts : sched) {
     dpc_tree_plan::Step st{};
     st.kind = ts.kind;
@@ -837,8 +831,8 @@ int dpc_tree_plan_create(const uint32_t* h_parent_slot, size_t ld, const uint64_
       const std::string why =
           ts.run.ring == 0 || ts.run.ring > max_ring
               ? std::string("ring larger than the kernel's LDS")
-              : tileplan::check_run(h_parent_slot, h_level_offsets, tileplan::limits_for(plan->threads, ts.run.ring),
-                                    ts.run);
+              : tileplan::check_run(h_parent_slot, h_level_offsets,
+                                    tileplan::limits_for(plan->threads, ts.run.ring, shape.last_steps), ts.run);
       if (!why.empty())
         return set_error(DPC_ERR_INTERNAL, "dpc_tree_plan_create: tile run of passes %zu-%zu: %s", ts.l, ts.r - 1,
                          why.c_str());

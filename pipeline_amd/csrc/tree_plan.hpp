@@ -79,9 +79,34 @@ struct Limits {
   uint32_t max_segs;  // pieces per tile (the kernel's LDS table)
 };
 
-inline Limits limits_for(uint32_t threads, uint32_t ring)
+inline Limits limits_for(uint32_t threads, uint32_t ring, uint32_t last_steps = 4)
 {
-  return Limits{threads, ring, threads * 4, 64};
+  return Limits{threads, ring, threads * last_steps, 64};
+}
+
+// The tiles' shape where the caller leaves it to the plan: threads of a workgroup,
+// and steps of the last pass's slots that a tile takes.
+//
+// Smaller workgroups split a tree over more CUs, shorten each tile's steps and mix the
+// reads of one tile with the writes of another; larger ones recompute fewer shared
+// ancestors.  Full propagation with 256 / 512 / 1024 threads: 10,000 nodes 5.9 / 5.9 /
+// 6.2 us, 50,000 7.1 / 7.1 / 7.2, 100,000 8.7 / 8.2 / 8.2, 250,007 12.7 / 11.7 / 11.9,
+// 500,000 15.8 / 15.1 / 15.8, 700,000 25.0 / 24.6 / 29.6 (1 % dirty 18.6 / 19.5 / 26.0),
+// 1,000,000 34.4 / 35.8 / 36.1.
+//
+// A shallow tree has all its nodes in the last pass, and tiles of four steps of them
+// leave a small one to a few CUs, whose steps follow each other: 20,000 nodes in two
+// passes are 20 tiles of five steps, 7.4 us, and 80 tiles of two, 5.0, with one step of
+// the last pass each (75,000: 7.9 -> 5.8; three passes: 7.9 -> 5.2; deeper trees, whose
+// tiles the ring bounds, unchanged).  In larger trees there are tiles enough, and
+// shorter ones recompute more ancestors (1,000,000 of few children 24.5 -> 34.0 us).
+struct Shape {
+  uint32_t threads, last_steps;
+};
+inline Shape default_shape(uint64_t slots)
+{
+  if (slots <= 75000) return Shape{256, 1};
+  return Shape{slots < 600000 ? 512u : 256u, 4};
 }
 
 struct Run {
@@ -455,7 +480,7 @@ struct Step {
 // resident together.
 inline std::vector<Step> schedule(const uint32_t* par, const uint64_t* off, size_t n, uint32_t threads,
                                   uint32_t max_ring, uint64_t capacity, uint64_t small_max, size_t small_levels_max,
-                                  size_t run_levels_max, uint32_t ring_step = 64)
+                                  size_t run_levels_max, uint32_t ring_step = 64, uint32_t last_steps = 4)
 {
   std::vector<Step> steps;
   const std::vector<uint8_t> link = links(par, off, n);
@@ -470,19 +495,19 @@ inline std::vector<Step> schedule(const uint32_t* par, const uint64_t* off, size
     bool done = false;
     for (size_t r = rmax; r >= l + 2 && !done; --r) {
       Step st{Step::kTiles, l, r, Run{}};
-      if (!build_run(par, off, l, r, limits_for(threads, max_ring), st.run)) continue;
+      if (!build_run(par, off, l, r, limits_for(threads, max_ring, last_steps), st.run)) continue;
       // the smallest ring that still fits the device in one wave of tiles
       uint32_t lo = 1, hi = max_ring / ring_step;  // ring = ring_step * k, k in [lo, hi]; hi is feasible
       if (st.run.tiles() <= capacity) {
         while (lo < hi) {
           const uint32_t mid = (lo + hi) / 2;
           Run trial;
-          if (build_run(par, off, l, r, limits_for(threads, ring_step * mid), trial) && trial.tiles() <= capacity)
+          if (build_run(par, off, l, r, limits_for(threads, ring_step * mid, last_steps), trial) && trial.tiles() <= capacity)
             hi = mid;
           else
             lo = mid + 1;
         }
-        if (ring_step * hi != max_ring) build_run(par, off, l, r, limits_for(threads, ring_step * hi), st.run);
+        if (ring_step * hi != max_ring) build_run(par, off, l, r, limits_for(threads, ring_step * hi, last_steps), st.run);
       }
       steps.push_back(std::move(st));
       l = r;
