@@ -5,12 +5,14 @@
 // (dp/culling/cpu/src/ManagerImpl.cpp:467-518), GroupCPU::updateOBBs (:114-162),
 // ManagerBitSet::calculateBoundingBox (dp/culling/src/ManagerBitSet.cpp:268-306)
 // and ResultBitSet::updateChanged (dp/culling/src/ResultBitSet.cpp:61-108).
+#include <algorithm>
 #include <atomic>
 #include <cfloat>
 #include <mutex>
 #include <type_traits>
 
 #include "cull_math.hpp"
+#include "cull_shape.hpp"
 #include "internal.hpp"
 #include "batch_types.hpp"
 
@@ -22,7 +24,7 @@ namespace {
 constexpr unsigned kCullThreads = 256;  // persistent streaming form
 constexpr unsigned kIndexedThreads = 512;  // plain form with an index array
 constexpr unsigned kPlainThreads = 1024;  // plain form without an index array
-constexpr unsigned kSmallThreads = 64;    // ... of short calls (launch_cull)
+constexpr unsigned kSmallThreads = 64;    // ... of short calls (flat_cull_threads)
 
 // With Diff (the cull of Manager::cull, which the result diff follows), the
 // wave that stores mask word w also stores the number of bits in which it
@@ -42,10 +44,11 @@ __device__ __forceinline__ uint8_t changed_in_word(unsigned long long old_bits, 
 // so every load of the wave is one contiguous 1 KiB (rows, box_a) or 512 B
 // (box_b) segment; the visibility bits leave as one ballot word per wave.
 // Without an index array every box and matrix is read once per launch, so
-// they are loaded as streaming data in 1024-thread blocks; with one (matrices
-// shared by several objects, e.g. the leaves of a transform tree), plain cached
-// loads in 512-thread blocks measured fastest (19.3 us against 19.5-19.7 us with
-// 256 threads for the 2.37M objects of a 1M-node tree).
+// they are loaded as streaming data, in blocks of 1024 threads or of one wave
+// (flat_cull_threads); with one (matrices shared by several objects, e.g. the
+// leaves of a transform tree), plain cached loads in 512-thread blocks measured
+// fastest (19.3 us against 19.5-19.7 us with 256 threads for the 2.37M objects of
+// a 1M-node tree; long calls take two tiles per wave, below).
 template <bool Indexed, bool Diff, unsigned Threads>
 __global__ __launch_bounds__(Threads) void cull_kernel(const float4* __restrict__ box_a,
                                                             const float2* __restrict__ box_b,
@@ -1024,17 +1027,13 @@ int launch_cull(const float* d_box_a, const float* d_box_b, const uint32_t* d_xf
       hipLaunchKernelGGL(kernel, dim3(grid_for(n_objects, threads)), dim3(threads), 0, s, a, b, d_xform, n_objects, p, ld, m,
                          out, old, count);
     };
-    // Without an index array, a workgroup of one wave in calls of up to 900,000
-    // objects: 10,000 objects in workgroups of 1024 threads occupy 10 CUs, sixteen
-    // waves each (the kernel: 10,000 objects 3.6 -> 2.8 us, 60,000 4.0 -> 3.2, 300,000
-    // 6.8 -> 5.6, 800,000 12.7 -> 12.1; two frames with their diffs over 300,000 21.4
-    // -> 19.3, 800,000 33.3 -> 31.4).  Longer calls wait for memory, and starting
-    // sixteen times as many workgroups costs more (1,048,576: 15.0 -> 15.7 us,
-    // 4,999,999: 65.3 -> 70.2).  With one, workgroups of 512 are spread well enough
-    // (two frames over 500,000, 4 to a matrix: 19.5 against 20.0).
+    // (with an index array workgroups of 512, whose loads wait for the indices first: two
+    // frames over 500,000 objects, 4 to a matrix, 19.5 us against 20.0 with one wave each;
+    // not measured below 500,000)
     if (d_xform)
       launch(cull_kernel<true, Diff, kIndexedThreads>, kIndexedThreads);
-    else if (n_objects <= 900'000)
+    else if (n_objects <= 100'000 ||  // (less than half a row: not worth asking for the device)
+             flat_cull_threads(n_objects, static_cast<uint32_t>(std::max(device_cu_count(), 1)), Diff) == kSmallThreads)
       launch(cull_kernel<false, Diff, kSmallThreads>, kSmallThreads);
     else
       launch(cull_kernel<false, Diff, kPlainThreads>, kPlainThreads);
