@@ -549,20 +549,38 @@ __global__ __launch_bounds__(kTreeThreads) void inverse_transpose_kernel(const f
 }
 
 // One bit per set byte.  A wave takes kBitsSlots consecutive slots and gathers
-// their bits in LDS, in a window of kBitsWindow bits from its lowest slot's index
-// on; each word that holds a bit goes to memory with one atomic.  What lies outside
-// gets a second window, and what lies outside that goes to memory bit by bit.
+// their bits in LDS, in a window of kBitsWindow bits from its lowest index on; each
+// word that holds a bit goes to memory with one atomic.  What lies outside gets a
+// second window, and what lies outside that goes to memory bit by bit, as do the bits
+// of a wave whose indices are in no order.
 // Slots are level-major and a level's indices ascend, so a wave's indices lie
 // close together (within a few of each other among leaves), in two places where a
 // level ends: a word then takes about one atomic per level instead of one per
 // slot.  What bounds it is those atomics: words are shared by waves on different
 // XCDs, whose L2s pass them to and fro, and a wave's atomics to one word follow
 // each other.  One atomic per set byte took 33.7 us for 700,000 set bytes and 9.9
-// us for 21,000 of 250,007; this takes 7.4 and 5.2.
+// us for 21,000 of 250,007; this takes 7.4 and 5.2.  In other orders than an ascending
+// one a window from the first slot's index on held little: 200,003 slots descending, all
+// set, took 22.2 us, and 5.1 from the lowest index on (one atomic per set byte: 18.8);
+// at random 13.3, and 11.6 without the windows (10.8).
 constexpr unsigned kBitsPerLane = 8;
 constexpr unsigned kBitsSlots = kWave * kBitsPerLane;
 constexpr unsigned kBitsWindow = 8192;
+constexpr unsigned kBitsBelow = 1024;
 static_assert(kBitsWindow == kWave * 4 * 32, "four window words per lane");
+
+// The wave's lowest value.
+__device__ __forceinline__ uint32_t wave_lowest(uint32_t v)
+{
+  auto lower = [&](uint32_t other) { v = other < v ? other : v; };
+  lower(__builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+  lower(__builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+  lower(__builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+  lower(__builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+  lower(__builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1 and 3
+  lower(__builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2 and 3
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), kWave - 1));
+}
 
 __global__ __launch_bounds__(kTreeThreads) void bytes_to_bits_kernel(const uint8_t* __restrict__ bytes,
                                                                      const uint32_t* __restrict__ index_of_slot,
@@ -589,24 +607,31 @@ __global__ __launch_bounds__(kTreeThreads) void bytes_to_bits_kernel(const uint8
     left[k] = index[k] < n_bits;
   }
   for (int pass = 0; pass < 2; ++pass) {
-    // the wave's first unwritten slot (the lowest index, where indices ascend)
-    size_t base = ~size_t(0);
+    // from the lowest unwritten index on (without a map the wave's first slot: one window holds them all)
+    bool any = false;
+    uint32_t lowest = 0xFFFFFFFFu;
 #pragma unroll
-    for (unsigned k = kBitsPerLane; k-- > 0;) {
-      const unsigned long long m = ballot(left[k]);
-      if (m == 0) continue;
-      const int from = __builtin_ctzll(m);
-      base = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(index[k]), from)) |
-             static_cast<size_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(index[k] >> 32), from))) << 32;
+    for (unsigned k = 0; k < kBitsPerLane; ++k) {
+      any |= left[k];
+      lowest = left[k] ? min(lowest, static_cast<uint32_t>(index[k])) : lowest;
     }
-    if (base == ~size_t(0)) return;
-    base &= ~size_t(31);
+    if (ballot(any) == 0) return;
+    size_t base = (index_of_slot ? static_cast<size_t>(wave_lowest(lowest)) : first) & ~size_t(31);
+    auto inside = [&](unsigned k) { return left[k] && index[k] - base < kBitsWindow; };
+    // The first 64 slots are asked whether they lie in it.  If few do, they may lie in
+    // another place together; if not, the indices are in no order.
+    const int asked = __popcll(ballot(left[0]));
+    if (4 * __popcll(ballot(inside(0))) < asked) {
+      const uint32_t at = __builtin_amdgcn_readlane(static_cast<int>(index[0]), __builtin_ctzll(ballot(left[0])));
+      base = (at > kBitsBelow ? at - kBitsBelow : 0) & ~31u;
+      if (4 * __popcll(ballot(inside(0))) < asked) break;
+    }
     windows[wave][lane] = make_uint4(0u, 0u, 0u, 0u);
     wave_lds_order();
 #pragma unroll
     for (unsigned k = 0; k < kBitsPerLane; ++k) {
-      const size_t at = index[k] - base;  // (an index below the base wraps to a large value)
-      if (left[k] && at < kBitsWindow) {
+      const size_t at = index[k] - base;
+      if (inside(k)) {
         atomicOr(&window[at >> 5], 1u << (at & 31));
         left[k] = false;
       }
