@@ -441,6 +441,14 @@ __global__ __launch_bounds__(256, K == 1 ? (Table ? 6 : 5) : K == 2 ? 4 : 2) voi
 // 32: 57 -> 39 us; 6,250 tiles x 20: 40 -> 32 us).
 
 constexpr uint32_t kServeViews = 64;  // frusta of a request, at most (dpc_server_submit)
+
+// A request of this many frusta or fewer takes the exact test: each of its tiles' object
+// bounds, for which the quick test reads the objects first, would serve one or two words
+// (quick -> exact: 10,000 x 1 6.1 -> 4.2 us, x 2 7.1 -> 4.2; 200,000 x 1 7.8 -> 5.7, x 2
+// 9.2 -> 7.3; 1,000,000 x 1 19.0 -> 17.5, x 2 20.8 -> 21.0).  Of four frusta the quick
+// test takes as long up to 100,000 objects (6.1 to 8.2 us, exact 5.3 to 8.0) and less
+// beyond (500,000 17.3 -> 15.1 us, 1,000,000 29.1 -> 22.4).
+constexpr uint32_t kFewFrusta = 2;
 static_assert(kServeViews <= kWave, "one lane per frustum");
 
 // A wave's current entry: its fields in the lanes of one register, each read where it
@@ -527,12 +535,12 @@ __global__ __launch_bounds__(256, 4) void cull_serve_kernel(const ServeEntry* __
   bool viewed = false;
   uint32_t waiting = 0, words = 0, exact = 0;
   for (;;) {
-    const uint32_t rest = e.pair_count() - first, count = rest < left ? rest : left;
+    const uint32_t listed = e.pair_count(), rest = listed - first, count = rest < left ? rest : left;
     const WorkItem item = serve_item<K>(e, tile, first, count);
     uint32_t done = 0, end = count;
     if (__builtin_expect(exact != 0, 0)) {
       --exact;
-    } else {
+    } else if (listed > kFewFrusta) {
       Slot slot[K];
       RawObj raw[K];
       load_objects<K>(scenes, item, lane, slot, raw);
@@ -938,7 +946,7 @@ int launch_copy_out(const void* d_copies, uint32_t n, const char* d_arena, uint6
   return check_launch("copy_out_kernel");
 }
 
-int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost, const void* d_pairs,
+int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost, uint64_t tiles, const void* d_pairs,
                  const void* d_scenes, const float* d_vps, uint64_t* d_masks, uint32_t objects_per_lane,
                  uint32_t waves_per_cu, void* stream_handle)
 {
@@ -949,11 +957,18 @@ int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost,
   // as a batch plan's lists are (dpc_batch_plan_create); a large one into as many
   // runs as the device holds waves: with a workgroup per CU more, a fifth of the equal
   // runs starts when the others end (1,000,003 objects x 32 views of which the quick
-  // test decides nothing: 307 us a tick, 282 without; ordinary 168 to 175, 168).
+  // test decides nothing: 307 us a tick, 282 without; ordinary 168 to 175, 168).  Up to
+  // that number each tile has a wave: with less than 16 frusta a run of 16 pairs passes
+  // over several tiles, and a wave has one tile's objects in flight at a time (500,000
+  // objects x 1 17.4 -> 13.1 us, 1,000,000 x 1 26.4 -> 18.9, x 4 22.6 -> 22.4).  Runs of
+  // one pair are for batches that take the exact test; the quick test reads the objects
+  // for two at least (10,000 x 2 5.6 -> 4.2 us).
   const uint64_t cus = device_cu_count();
   const uint32_t held = waves_per_block * (objects_per_lane == 2 ? kServeBlocks<2> : kServeBlocks<1>);
   uint64_t waves = cus * (waves_per_cu ? waves_per_cu : held);
-  waves = std::min(waves, total_cost / std::clamp<uint64_t>((total_cost + 5 * cus - 1) / (5 * cus), 2, 16));
+  const uint64_t run =
+      std::clamp<uint64_t>((total_cost + 5 * cus - 1) / (5 * cus), total_cost <= kFewFrusta * tiles ? 1 : 2, 16);
+  waves = std::min(waves, std::max(total_cost / run, tiles));
   if (waves == 0) waves = 1;
   const uint64_t blocks = (waves + waves_per_block - 1) / waves_per_block;
   const auto* e = static_cast<const ServeEntry*>(d_entries);

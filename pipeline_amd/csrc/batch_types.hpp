@@ -27,8 +27,9 @@ struct ServeEntry {
 };
 static_assert(sizeof(ServeEntry) == 32, "ServeEntry layout");
 
-// Launches one serving batch; every pointer is device memory.
-int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost, const void* d_pairs,
+// Launches one serving batch; every pointer is device memory.  total_cost is the sum of
+// the entries' tiles times frusta, tiles that of their tiles.
+int launch_serve(const void* d_entries, uint32_t n_entries, uint64_t total_cost, uint64_t tiles, const void* d_pairs,
                  const void* d_scenes, const float* d_vps, uint64_t* d_masks, uint32_t objects_per_lane,
                  uint32_t waves_per_cu, void* stream);
 

@@ -496,7 +496,7 @@ void dpc_server::issue_batch(StreamSlot& slot)
   uint32_t n_copies = 0;
   uint64_t copy_words = 0;
   std::vector<uint64_t> mask_off(pick.size());  // byte offset of each request's masks in the device arena
-  uint64_t cost = 0, mask_word = 0, tests = 0;
+  uint64_t cost = 0, tiles = 0, mask_word = 0, tests = 0;
   uint32_t p = 0;
   for (size_t k = 0; k < pick.size(); ++k) {
     const Request& r = *pick[k];
@@ -509,6 +509,7 @@ void dpc_server::issue_batch(StreamSlot& slot)
     en.cost_begin = cost;
     en.objects = sc.n;
     cost += static_cast<uint64_t>(en.tiles) * r.n_frusta;
+    tiles += en.tiles;
     mask_off[k] = masks_off + 8 * mask_word;
     for (uint32_t f = 0; f < r.n_frusta; ++f, ++p) {
       pairs[p].frustum = p;
@@ -605,7 +606,7 @@ void dpc_server::issue_batch(StreamSlot& slot)
   }
   t_part[3] = now();
   if (rc == DPC_OK) {
-    rc = dpc::launch_serve(slot.d_arena + entries_off, static_cast<uint32_t>(pick.size()), cost,
+    rc = dpc::launch_serve(slot.d_arena + entries_off, static_cast<uint32_t>(pick.size()), cost, tiles,
                            slot.d_arena + pairs_off, d_scene_table, reinterpret_cast<const float*>(slot.d_arena + vps_off),
                            reinterpret_cast<uint64_t*>(slot.d_arena + masks_off), K, cfg.waves_per_cu, s);
   }

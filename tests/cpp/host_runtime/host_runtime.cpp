@@ -150,7 +150,7 @@ int set_error(int code, const char* fmt, ...)
   va_end(ap);
   return code;
 }
-int launch_serve(const void*, uint32_t, uint64_t, const void*, const void*, const float*, uint64_t*, uint32_t,
+int launch_serve(const void*, uint32_t, uint64_t, uint64_t, const void*, const void*, const float*, uint64_t*, uint32_t,
                  uint32_t, void*)
 {
   return DPC_OK;
