@@ -39,6 +39,7 @@
 
 #include "../batch_types.hpp"
 #include "dpcull_hip.h"
+#include "highest.hpp"
 #include "trace.hpp"
 
 namespace dpc {
@@ -972,8 +973,7 @@ int dpc_server_submit(dpc_server* s, uint32_t scene_id, const float* vps, uint32
     }
   }
   // the largest delta index, found before the lock is taken
-  uint32_t top = 0;
-  for (uint32_t k = 0; k < n_delta; ++k) top = std::max(top, didx[k]);
+  const uint32_t top = dpc::highest_index(didx, n_delta);
   std::lock_guard<std::mutex> g(s->mu);
   // (a scene still being uploaded has no id for its caller yet, and no sizes)
   if (scene_id >= s->scenes.size() || !s->scenes[scene_id].live || !s->scenes[scene_id].ready)
