@@ -56,10 +56,12 @@ struct StageJob {
 };
 static_assert(sizeof(StageJob) == 32, "StageJob layout");
 
-// Scatters the n jobs' deltas out of an arena of `bytes` bytes (below 2^31).  With
+// Scatters the n jobs' deltas out of an arena of `bytes` bytes (below 2^31), in one
+// launch; the jobs travel by value in its arguments, at most kStageJobs.  With
 // d_arena set the arena lies in pinned host memory and its first desc_bytes bytes
 // (a multiple of 16) are copied to d_arena as well: a batch's whole upload in one
 // launch.  With d_arena null it is device memory, and the deltas are scattered only.
+constexpr uint32_t kStageJobs = 64;
 int launch_stage(const char* arena, uint64_t bytes, char* d_arena, uint64_t desc_bytes, const StageJob* jobs, uint32_t n,
                  void* stream);
 

@@ -249,7 +249,6 @@ __global__ __launch_bounds__(256) void scatter_host_kernel(float4* __restrict__ 
 // launch that reads the host's arena itself has neither.  One request for each of
 // 16 scenes: 428 to 436 us a tick with a copy and scatters, 382 to 396 with this.
 constexpr uint32_t kStageChunk = 192;
-constexpr uint32_t kStageJobs = 64;  // jobs of one launch, by value
 // 16 workgroups of 13 KB in flight fill PCIe (1 MB: 32 us with 16, 37 with 64 or
 // more, of which 11 are a launch and its completion).
 constexpr uint32_t kStageHostBlocks = 16;
@@ -1142,8 +1141,8 @@ int launch_scatter_host(float* d_planes, size_t ld, const uint32_t* idx, const f
 int launch_stage(const char* arena, uint64_t bytes, char* d_arena, uint64_t desc_bytes, const StageJob* jobs, uint32_t n,
                  void* stream)
 {
-  if (!arena || (n && !jobs) || bytes >= (1ull << 31) || desc_bytes > bytes || desc_bytes % 16 || !aligned(arena, 16) ||
-      !aligned(d_arena, 16) || (desc_bytes && !d_arena))
+  if (!arena || (n && !jobs) || n > kStageJobs || bytes >= (1ull << 31) || desc_bytes > bytes || desc_bytes % 16 ||
+      !aligned(arena, 16) || !aligned(d_arena, 16) || (desc_bytes && !d_arena))
     return set_error(DPC_ERR_INVALID_ARGUMENT, "launch_stage: bad argument");
   for (uint32_t k = 0; k < n; ++k) {
     const StageJob& j = jobs[k];
@@ -1155,28 +1154,24 @@ int launch_stage(const char* arena, uint64_t bytes, char* d_arena, uint64_t desc
   StageJobs args;
   args.desc_chunks = static_cast<uint32_t>(desc_bytes / 16);
   args.desc_units = (args.desc_chunks + kStageChunk - 1) / kStageChunk;
-  for (uint32_t k = 0; k < n || args.desc_units;) {
-    args.n = 0;
-    args.units = args.desc_units;
-    for (; k < n && args.n < kStageJobs; ++k) {
-      if (jobs[k].count == 0) continue;
-      args.job[args.n] = jobs[k];
-      args.first_unit[args.n++] = args.units;
-      args.units += (jobs[k].count + 63) / 64;
-    }
-    if (args.units == 0) break;
-    const uint32_t most = d_arena ? kStageHostBlocks : 8u * static_cast<uint32_t>(device_cu_count());
-    const dim3 grid(std::min((args.units + 3) / 4, most));
-    if (d_arena)
-      hipLaunchKernelGGL(stage_kernel<true>, grid, dim3(256), 0, as_stream(stream), arena, static_cast<uint32_t>(bytes),
-                         reinterpret_cast<u32x4_t*>(d_arena), args);
-    else
-      hipLaunchKernelGGL(stage_kernel<false>, grid, dim3(256), 0, as_stream(stream), arena, static_cast<uint32_t>(bytes),
-                         nullptr, args);
-    if (int rc = check_launch("stage_kernel")) return rc;
-    args.desc_chunks = args.desc_units = 0;
+  args.n = 0;
+  args.units = args.desc_units;
+  for (uint32_t k = 0; k < n; ++k) {
+    if (jobs[k].count == 0) continue;
+    args.job[args.n] = jobs[k];
+    args.first_unit[args.n++] = args.units;
+    args.units += (jobs[k].count + 63) / 64;
   }
-  return DPC_OK;
+  if (args.units == 0) return DPC_OK;
+  const uint32_t most = d_arena ? kStageHostBlocks : 8u * static_cast<uint32_t>(device_cu_count());
+  const dim3 grid(std::min((args.units + 3) / 4, most));
+  if (d_arena)
+    hipLaunchKernelGGL(stage_kernel<true>, grid, dim3(256), 0, as_stream(stream), arena, static_cast<uint32_t>(bytes),
+                       reinterpret_cast<u32x4_t*>(d_arena), args);
+  else
+    hipLaunchKernelGGL(stage_kernel<false>, grid, dim3(256), 0, as_stream(stream), arena, static_cast<uint32_t>(bytes),
+                       nullptr, args);
+  return check_launch("stage_kernel");
 }
 
 }  // namespace dpc

@@ -50,6 +50,7 @@ namespace {
 
 constexpr uint32_t kMaxScenes = 64;
 constexpr uint32_t kMaxBatch = 64;
+static_assert(kMaxBatch <= dpc::kStageJobs, "one launch scatters a batch's deltas");
 constexpr uint32_t kMaxFrusta = 64;
 // the pinned staging area of one batch's descriptors (entries, pairs, frusta, copy-outs)
 constexpr uint64_t kHostArena = 4096 + kMaxBatch * 32 + kMaxBatch * kMaxFrusta * (16 + 64) + kMaxBatch * 32 + 4 * 256;
