@@ -18,9 +18,9 @@
 // vector instructions with the quick test's products on the vector unit, 190 when
 // each pair took the exact test).  500,003 objects x 32 frusta: 109 us with the
 // exact test, 35 with the quick test, 26 with its products on the matrix cores, of
-// which 9 are reading the objects and 11 the instructions; 64 frusta over 64 groups
-// of 2,097,152 objects: 40 -> 35 us, 4.6 TB/s, bound by reading the objects, those
-// of undecided pairs twice.
+// which 9 are reading the objects and 11 the instructions, and 68 where the quick test
+// decides nothing (kDenseLanes); 64 frusta over 64 groups of 2,097,152 objects: 40 ->
+// 35 us, 5.3 TB/s, bound by reading the objects, those of undecided pairs twice.
 //
 // Schedule: items are sorted by cost (frusta x objects) on the host, and the
 // persistent grid walks them round-robin (wave w takes w, w+W, ...), which
